@@ -115,10 +115,10 @@ enum TileCfg : int32_t {
   kTile32x32 = 1,  // 64 threads, 1 wave of 32x32
   kTile64x32 = 2,  // 128 threads, 2 waves of 32x32
   kTile128x64 = 3, // 512 threads, 8 waves of 32x32
-  // the same tiles with three real MFMAs per complex product (3M)
-  kTile64x64_3M = 4,
-  kTile32x32_3M = 5,
-  kTile128x64_3M = 6,
+  // three real MFMAs per complex product (3M)
+  kTile64x64_3M = 4,   // 256 threads; up to 64x64: the launch takes a smaller tile where that is faster
+  kTile32x32_3M = 5,   // 256 threads, 4 waves of 16x16
+  kTile128x64_3M = 6,  // 512 threads, 8 waves of 32x32
   kNumTileCfgs = 7
 };
 int tile_m(int cfg);
@@ -141,6 +141,9 @@ __device__ inline int xcd_remap(int w, int total) {
 // Host-side launchers (defined in the .hip translation units).
 hipError_t launch_zgemm(const ZGroup& g, int cfg, hipStream_t stream);
 hipError_t launch_zgemm_update(const ZGroup& g, int cfg, hipStream_t stream);
+// The inversion's updates of one panel's columns (op = N, alpha = 1): 32x32
+// tiles, four MFMAs per complex product.
+hipError_t launch_zgemm_narrow(const ZGroup& g, hipStream_t stream);
 // Same problems, products computed in complex64 on FP32 matrix cores.
 hipError_t launch_zgemm_f32(const ZGroup& g, int cfg, hipStream_t stream);
 

@@ -2,13 +2,12 @@
 //
 // Each launch carries up to kMaxProblems independent problems
 //   D = sum_t alpha_t op(A_t) op(B_t) + sum_a (c1_a F_a + c2_a F_a^H)
-// over nE energies.  Complex products are four real MFMAs
-// (v_mfma_f64_16x16x4f64): re += ar*br - ai*bi, im += ar*bi + ai*br; or,
-// in the 3M configurations, three: P1 = ar*br, P2 = ai*bi and
-// P3 = (ar + ai)(br + bi) accumulate separately and re = P1 - P2,
-// im = P3 - P1 - P2 in the epilogue (25% fewer matrix-core operations, one
-// more accumulator set, two FP64 adds per fragment pair).
-// Tiles of op(A) (TM x TK) and op(B) (TK x TN) are staged through LDS,
+// over nE energies.  Two kernels:
+//  * zgemm3m_kernel (second half of the file), the FP64 products of the
+//    sweeps: three real MFMAs per complex product;
+//  * zgemm_grouped_kernel: four real MFMAs (v_mfma_f64_16x16x4f64),
+//    re += ar*br - ai*bi, im += ar*bi + ai*br, in FP64 or with FP32 operands.
+// In zgemm_grouped_kernel, tiles of op(A) (TM x TK) and op(B) (TK x TN) are staged through LDS,
 // k-major so that every MFMA fragment read is 16 contiguous complex values;
 // conjugation and alpha are applied while staging, so the inner loop is the
 // same for every op combination.  Global loads are issued for the next k-tile
@@ -30,16 +29,12 @@ constexpr int PAD = 1;
 // instead of 16.9 KB) does not cap the number of workgroups per CU below what
 // its registers allow (measured: equal at b = 32, +13-34% at b = 48); FP32
 // products, whose MFMAs take half as long, lose more to the extra barriers
-// than they gain and keep the deeper stage.  kTKo overrides the depth: the
-// 3M 128x64 tile (one workgroup per CU by its registers either way) stages
-// k = 16, so that each stage's MFMAs cover the next stage's global-load
-// latency and the barrier count halves (measured 2-4% faster than k = 8 at
-// b = 128-512; the same depth made the 4M 128x64 and the 3M 64x64 tiles
-// slower: 99 KB and 66 KB of LDS cost them workgroups per CU).
-template <int TM, int TN, bool kF32 = false, int kTKo = 0>
+// than they gain and keep the deeper stage (k = 16 made the 4M 128x64 tile
+// slower: 99 KB of LDS cost it a workgroup per CU).
+template <int TM, int TN, bool kF32 = false>
 struct TileShape {
   static constexpr bool kSmall = TM == 32 && TN == 32 && !kF32;
-  static constexpr int kTK = kTKo ? kTKo : (kSmall ? 4 : 8);
+  static constexpr int kTK = kSmall ? 4 : 8;
   static constexpr int kSlab = kSmall ? 16 : 32;
   static constexpr int kWavesM = TM / 32;
   static constexpr int kWavesN = TN / 32;
@@ -48,10 +43,10 @@ struct TileShape {
   static constexpr int kBPer = kTK * TN / kThreads;
 };
 
-template <int TM, int TN, bool F32, int TKo>
+template <int TM, int TN, bool F32>
 __device__ inline void load_a(const ZTerm& t, int e, int m, int m0, int k0, int tid,
-                              double2 (&ra)[TileShape<TM, TN, F32, TKo>::kAPer]) {
-  using S = TileShape<TM, TN, F32, TKo>;
+                              double2 (&ra)[TileShape<TM, TN, F32>::kAPer]) {
+  using S = TileShape<TM, TN, F32>;
   const double2* A = t.A + (int64_t)e * t.sA;
   const double2 zero = cmk(0.0, 0.0);
 #pragma unroll
@@ -72,11 +67,11 @@ __device__ inline void load_a(const ZTerm& t, int e, int m, int m0, int k0, int 
 __device__ inline void put(double2* p, double2 v) { *p = v; }
 __device__ inline void put(float2* p, double2 v) { *p = make_float2((float)v.x, (float)v.y); }
 
-template <int TM, int TN, bool F32, int TKo, typename LT>
+template <int TM, int TN, bool F32, typename LT>
 __device__ inline void store_a(const ZTerm& t, int tid,
-                               const double2 (&ra)[TileShape<TM, TN, F32, TKo>::kAPer],
+                               const double2 (&ra)[TileShape<TM, TN, F32>::kAPer],
                                LT (*As)[TM + PAD]) {
-  using S = TileShape<TM, TN, F32, TKo>;
+  using S = TileShape<TM, TN, F32>;
   const bool cj = (t.opA == kOpC);
 #pragma unroll
   for (int i = 0; i < S::kAPer; ++i) {
@@ -90,10 +85,10 @@ __device__ inline void store_a(const ZTerm& t, int tid,
   }
 }
 
-template <int TM, int TN, bool F32, int TKo>
+template <int TM, int TN, bool F32>
 __device__ inline void load_b(const ZTerm& t, int e, int n, int n0, int k0, int tid,
-                              double2 (&rb)[TileShape<TM, TN, F32, TKo>::kBPer]) {
-  using S = TileShape<TM, TN, F32, TKo>;
+                              double2 (&rb)[TileShape<TM, TN, F32>::kBPer]) {
+  using S = TileShape<TM, TN, F32>;
   const double2* B = t.B + (int64_t)e * t.sB;
   const double2 zero = cmk(0.0, 0.0);
 #pragma unroll
@@ -111,11 +106,11 @@ __device__ inline void load_b(const ZTerm& t, int e, int n, int n0, int k0, int 
   }
 }
 
-template <int TM, int TN, bool F32, int TKo, typename LT>
+template <int TM, int TN, bool F32, typename LT>
 __device__ inline void store_b(const ZTerm& t, int tid,
-                               const double2 (&rb)[TileShape<TM, TN, F32, TKo>::kBPer],
+                               const double2 (&rb)[TileShape<TM, TN, F32>::kBPer],
                                LT (*Bs)[TN + PAD]) {
-  using S = TileShape<TM, TN, F32, TKo>;
+  using S = TileShape<TM, TN, F32>;
   const bool cj = (t.opB == kOpC);
 #pragma unroll
   for (int i = 0; i < S::kBPer; ++i) {
@@ -129,9 +124,9 @@ __device__ inline void store_b(const ZTerm& t, int tid,
   }
 }
 
-template <int TM, int TN, typename LT, int TKo>
+template <int TM, int TN, typename LT>
 struct Smem {
-  using S = TileShape<TM, TN, std::is_same<LT, float2>::value, TKo>;
+  using S = TileShape<TM, TN, std::is_same<LT, float2>::value>;
   static constexpr int kA = S::kTK * (TM + PAD);  // one LDS stage of op(A), k-major (LT elements)
   static constexpr int kB = S::kTK * (TN + PAD);  // one LDS stage of op(B), k-major
   static constexpr int kMainBytes = (2 * kA + 2 * kB) * (int)sizeof(LT);
@@ -155,18 +150,14 @@ __device__ inline double4_t mfma_nega(double a, double b, double4_t c) {
 // addends and stores stay complex128 (the mixed-precision sweeps).
 // Occupancy target: four 64x64 workgroups per CU (33 KB LDS each, <= 128
 // VGPRs), measured faster than three.
-// k3M: FP64 products by three real MFMAs per complex product (see the file
-// header); the extra accumulator set lowers the 64x64 target to three
-// workgroups per CU.
-template <int TM, int TN, int kRole, bool kF32, bool k3M = false, int kTKo = 0>
-__global__ void __launch_bounds__((TileShape<TM, TN, kF32, kTKo>::kThreads),
-                                  (TM * TN > 4096 ? 1 : (TM * TN == 4096 ? (k3M ? 3 : 4) : 2)))
+template <int TM, int TN, int kRole, bool kF32>
+__global__ void __launch_bounds__((TileShape<TM, TN, kF32>::kThreads),
+                                  (TM * TN > 4096 ? 1 : (TM * TN == 4096 ? 4 : 2)))
 zgemm_grouped_kernel(const ZGroup g) {
-  static_assert(!(k3M && kF32), "3M products are built for FP64 only");
-  using S = TileShape<TM, TN, kF32, kTKo>;
+  using S = TileShape<TM, TN, kF32>;
   using LT = typename std::conditional<kF32, float2, double2>::type;
   using AccT = typename std::conditional<kF32, float4_t, double4_t>::type;
-  using L = Smem<TM, TN, LT, kTKo>;
+  using L = Smem<TM, TN, LT>;
   constexpr int TK = S::kTK;
   constexpr int kSlab = S::kSlab;
   __shared__ __align__(16) char smem_raw[L::kBytes];
@@ -198,15 +189,13 @@ zgemm_grouped_kernel(const ZGroup g) {
   const int wm = wave / S::kWavesN;
   const int wn = wave % S::kWavesN;
 
-  // 4M: accr = re, acci = im.  3M: accr = P1, acci = P2, accs = P3.
-  AccT accr[2][2], acci[2][2], accs[k3M ? 2 : 1][k3M ? 2 : 1];
+  AccT accr[2][2], acci[2][2];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       accr[i][j] = AccT{0, 0, 0, 0};
       acci[i][j] = AccT{0, 0, 0, 0};
-      if constexpr (k3M) accs[i][j] = AccT{0, 0, 0, 0};
     }
 
   for (int ti = 0; ti < P.nterms; ++ti) {
@@ -215,17 +204,17 @@ zgemm_grouped_kernel(const ZGroup g) {
     const ZTerm T = P.t[ti];
     const int nk = (T.k + TK - 1) / TK;
     double2 ra[S::kAPer], rb[S::kBPer];
-    load_a<TM, TN, kF32, kTKo>(T, e, m, m0, 0, tid, ra);
-    load_b<TM, TN, kF32, kTKo>(T, e, n, n0, 0, tid, rb);
-    store_a<TM, TN, kF32, kTKo, LT>(T, tid, ra, As(0));
-    store_b<TM, TN, kF32, kTKo, LT>(T, tid, rb, Bs(0));
+    load_a<TM, TN, kF32>(T, e, m, m0, 0, tid, ra);
+    load_b<TM, TN, kF32>(T, e, n, n0, 0, tid, rb);
+    store_a<TM, TN, kF32, LT>(T, tid, ra, As(0));
+    store_b<TM, TN, kF32, LT>(T, tid, rb, Bs(0));
     __syncthreads();
     for (int kt = 0; kt < nk; ++kt) {
       const int cur = kt & 1;
       const bool more = (kt + 1 < nk);
       if (more) {
-        load_a<TM, TN, kF32, kTKo>(T, e, m, m0, (kt + 1) * TK, tid, ra);
-        load_b<TM, TN, kF32, kTKo>(T, e, n, n0, (kt + 1) * TK, tid, rb);
+        load_a<TM, TN, kF32>(T, e, m, m0, (kt + 1) * TK, tid, ra);
+        load_b<TM, TN, kF32>(T, e, n, n0, (kt + 1) * TK, tid, rb);
       }
       auto as = As(cur);
       auto bs = Bs(cur);
@@ -237,17 +226,8 @@ zgemm_grouped_kernel(const ZGroup g) {
       for (int j = 0; j < 2; ++j) fb[0][j] = bs[lane >> 4][wn * 32 + j * 16 + (lane & 15)];
 #pragma unroll
       for (int ks = 0; ks < TK / 4; ++ks) {
-        // 3M: no fragment prefetch (its registers hold the third accumulator set)
-        const int c = k3M ? 0 : (ks & 1);
-        if constexpr (k3M) {
-          if (ks > 0) {
-            const int kk = ks * 4 + (lane >> 4);
-#pragma unroll
-            for (int i = 0; i < 2; ++i) fa[0][i] = as[kk][wm * 32 + i * 16 + (lane & 15)];
-#pragma unroll
-            for (int j = 0; j < 2; ++j) fb[0][j] = bs[kk][wn * 32 + j * 16 + (lane & 15)];
-          }
-        } else if (ks + 1 < TK / 4) {
+        const int c = ks & 1;
+        if (ks + 1 < TK / 4) {
           const int kk = (ks + 1) * 4 + (lane >> 4);
 #pragma unroll
           for (int i = 0; i < 2; ++i) fa[c ^ 1][i] = as[kk][wm * 32 + i * 16 + (lane & 15)];
@@ -278,24 +258,6 @@ zgemm_grouped_kernel(const ZGroup g) {
 #pragma unroll
             for (int j = 0; j < 2; ++j)
               acci[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[c][i].y, fb[c][j].x, acci[i][j], 0, 0, 0);
-        } else if constexpr (k3M) {
-          double sa[2], sb[2];
-#pragma unroll
-          for (int i = 0; i < 2; ++i) sa[i] = fa[c][i].x + fa[c][i].y;
-#pragma unroll
-          for (int j = 0; j < 2; ++j) sb[j] = fb[c][j].x + fb[c][j].y;
-#pragma unroll
-          for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) accr[i][j] = mfma(fa[c][i].x, fb[c][j].x, accr[i][j]);
-#pragma unroll
-          for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) acci[i][j] = mfma(fa[c][i].y, fb[c][j].y, acci[i][j]);
-#pragma unroll
-          for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) accs[i][j] = mfma(sa[i], sb[j], accs[i][j]);
         } else {
 #pragma unroll
           for (int i = 0; i < 2; ++i)
@@ -316,8 +278,8 @@ zgemm_grouped_kernel(const ZGroup g) {
         }
       }
       if (more) {
-        store_a<TM, TN, kF32, kTKo, LT>(T, tid, ra, As(cur ^ 1));
-        store_b<TM, TN, kF32, kTKo, LT>(T, tid, rb, Bs(cur ^ 1));
+        store_a<TM, TN, kF32, LT>(T, tid, ra, As(cur ^ 1));
+        store_b<TM, TN, kF32, LT>(T, tid, rb, Bs(cur ^ 1));
       }
       __syncthreads();
     }
@@ -349,13 +311,8 @@ zgemm_grouped_kernel(const ZGroup g) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const int rr = kF32 ? ((lane >> 4) * 4 + r) : (r * 4 + (lane >> 4));
-            if constexpr (k3M) {
-              const double p1 = accr[i][j][r], p2 = acci[i][j][r];
-              Cs[ri + rr][wn * 32 + j * 16 + (lane & 15)] = cmk(p1 - p2, accs[i][j][r] - p1 - p2);
-            } else {
-              Cs[ri + rr][wn * 32 + j * 16 + (lane & 15)] =
-                  cmk((double)accr[i][j][r], (double)acci[i][j][r]);
-            }
+            Cs[ri + rr][wn * 32 + j * 16 + (lane & 15)] =
+                cmk((double)accr[i][j][r], (double)acci[i][j][r]);
           }
       }
     }
@@ -425,7 +382,7 @@ zgemm_grouped_kernel(const ZGroup g) {
   }
 }
 
-template <int TM, int TN, int kRole, bool kF32 = false, bool k3M = false, int kTKo = 0>
+template <int TM, int TN, int kRole, bool kF32 = false>
 hipError_t launch_cfg(const ZGroup& g0, hipStream_t stream) {
   ZGroup g = g0;
   int per = 0;  // workgroups per energy (all problems)
@@ -440,9 +397,434 @@ hipError_t launch_cfg(const ZGroup& g0, hipStream_t stream) {
   const int64_t total = (int64_t)per * g.nE;
   if (total == 0) return hipSuccess;
   if (total > 0x7fffffff) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((zgemm_grouped_kernel<TM, TN, kRole, kF32, k3M, kTKo>), dim3((unsigned)total),
-                     dim3(TileShape<TM, TN, kF32, kTKo>::kThreads), 0, stream, g);
+  hipLaunchKernelGGL((zgemm_grouped_kernel<TM, TN, kRole, kF32>), dim3((unsigned)total),
+                     dim3(TileShape<TM, TN, kF32>::kThreads), 0, stream, g);
   return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// FP64 products of the sweeps: three real MFMAs per complex product
+// ---------------------------------------------------------------------------
+//
+// P1 = ar br, P2 = ai bi and P3 = (ar + ai)(br + bi) accumulate in three
+// accumulator sets; re = P1 - P2, im = P3 - P1 - P2 in the epilogue.  Bound by
+// the matrix cores: v_mfma_f64_16x16x4f64 takes 64 cycles of its SIMD, and every
+// vector instruction takes its issue cycles from the same pipe (measured with
+// twelve independent MFMAs in a loop: 64.4 cycles per MFMA alone; each FP64 add
+// in the loop costs 7.8 cycles of MFMA time, each 32-bit VALU instruction or
+// LDS access about 3).  So the loop holds almost nothing but MFMAs:
+//  * alpha = +-1 and the conjugations never touch an operand.  A conjugated
+//    operand changes the sign with which its imaginary part enters the two
+//    fragment sums (an fma with a scalar +-1 in the place of the add) and the
+//    sign of P2, and a negative term that of all three; the accumulators keep
+//    the sum up to those signs, are negated where a term's signs differ from
+//    the one before it, and the last signs are applied in the epilogue.  Any
+//    other alpha scales op(A) on its way into LDS (kGeneral).
+//  * operands come by buffer loads with one lane offset per element and a scalar
+//    offset per k-tile; rows and columns beyond the edge have an offset beyond
+//    the buffer, which reads as zero, and so have the inner indices beyond K
+//    (kTail: K not a multiple of 8 costs a compare and a select per element).
+//  * two k-tiles per loop pass, so that every LDS address is a constant offset.
+//  * the reads of the next k-step's fragments, the stores of the next k-tile and
+//    the loads of the one after it sit between the MFMAs (scheduled by
+//    sched_group_barrier), with one barrier per k-tile, placed between its two
+//    k-steps: what is read after it was stored a whole k-step before.
+// The epilogue works on the accumulators: register r of a lane holds D[4 r +
+// lane / 16][lane % 16] of its 16 x 16 tile, so a store covers four rows of
+// 256 contiguous bytes; no LDS pass, no barrier.  Waves whose part of the tile lies beyond the
+// matrix only help to stage.
+// Measured (MI355X, TFLOP/s by 8 m n k, against the kernel it replaced, which
+// staged its epilogue through LDS, waited for its own LDS traffic and relied on
+// a third workgroup per CU): 256^3 x 512 energies 89 (76), 512^3 x 16 94 (76),
+// 256^3 x 8 80 (48), 208^3 x 64 73 (49), 96^3 x 64 67 (36), 91 x 77 x 65 x 48
+// 33 (17); results are bit for bit the same.  90% of the time the matrix cores
+// are busy at 512^3; the rest is the FP64 adds of the fragment sums (5%) and
+// the epilogue.  Two waves per SIMD at 64 x 64 (256 registers) beat three (168,
+// spilled: 76).
+#define QX_SGB(mask, n) __builtin_amdgcn_sched_group_barrier(mask, n, 0)
+constexpr int kSgMfma = 0x8, kSgVmemRead = 0x20, kSgDsRead = 0x100, kSgDsWrite = 0x200;
+
+typedef unsigned uint4_t __attribute__((ext_vector_type(4)));
+constexpr unsigned kOob = 0x80000000u;  // beyond num_records: loads give 0, stores are dropped
+__device__ inline __amdgpu_buffer_rsrc_t buf_of(const void* p) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, 0x7fffffff, 0x00020000);
+}
+__device__ inline double2 buf_load(__amdgpu_buffer_rsrc_t r, unsigned off, unsigned soff) {
+  return __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(r, off, soff, 0));
+}
+__device__ inline void buf_store(__amdgpu_buffer_rsrc_t r, unsigned off, double2 v) {
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4_t, v), r, off, 0, 0);
+}
+
+// kFast: alpha = +-1, every K a multiple of 8; kFastTail: alpha = +-1;
+// kGeneral: any.  kPlain4M: four MFMAs per product (no conjugation, alpha = 1).
+enum Form : int { kFast = 0, kFastTail = 1, kGeneral = 2, kPlain4M = 3 };
+
+template <int TM, int TN, int WM, int WN>
+struct Tile3M {
+  static constexpr int kTK = 8;
+  static constexpr int kThreads = 64 * WM * WN;
+  static constexpr int SI = TM / WM / 16, SJ = TN / WN / 16;  // 16 x 16 tiles of a wave
+  static constexpr int kAPer = TM * kTK / kThreads, kBPer = kTK * TN / kThreads;
+  static constexpr int LA = TM + 1, LB = TN + 1;
+};
+
+// TM x TN output tile, WM x WN waves, at least MINW waves per SIMD.  kRole only
+// separates kernel names in traces: 0 = sweep products, 1 = trailing updates
+// inside the blocked inversion.
+template <int TM, int TN, int WM, int WN, int MINW, int kRole, int kForm>
+__global__ void __launch_bounds__(64 * WM * WN, MINW) zgemm3m_kernel(const ZGroup g) {
+  using S = Tile3M<TM, TN, WM, WN>;
+  constexpr int SI = S::SI, SJ = S::SJ, TK = S::kTK;
+  constexpr bool kGen = kForm == kGeneral, kTail = kForm != kFast, k4M = kForm == kPlain4M;
+  __shared__ double2 lds_a[2 * TK * S::LA];
+  __shared__ double2 lds_b[2 * TK * S::LB];
+
+  const int per = g.wg_base[g.nprob];
+  const int wid = xcd_remap(blockIdx.x, per * g.nE);
+  const int e = wid / per;
+  const int rem = wid - e * per;
+  int p = 0;
+  while (p + 1 < g.nprob && rem >= g.wg_base[p + 1]) ++p;
+  const ZProblem& P = g.p[p];
+  const int tt = rem - g.wg_base[p];
+  const int m0 = (tt / g.tiles_n[p]) * TM;
+  const int n0 = (tt % g.tiles_n[p]) * TN;
+  const int m = P.m, n = P.n;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  const int l16 = lane & 15, kq = lane >> 4;
+  const int mw = m0 + wm * (16 * SI), nw = n0 + wn * (16 * SJ);
+  const bool some = mw < m && nw < n;  // this wave has valid outputs
+
+  // `live` waves multiply, the others only stage (two copies of the code, so
+  // that the copy without MFMAs does not weigh on the other's registers)
+  auto body = [&](auto live) {
+  constexpr bool kLive = decltype(live)::value;
+  double4_t acc1[SI][SJ], acc2[SI][SJ], acc3[SI][SJ];
+#pragma unroll
+  for (int i = 0; i < SI; ++i)
+#pragma unroll
+    for (int j = 0; j < SJ; ++j) acc1[i][j] = acc2[i][j] = acc3[i][j] = double4_t{0, 0, 0, 0};
+
+  double2 ra[S::kAPer], rb[S::kBPer];
+  double2 fa[2][SI], fb[2][SJ];
+  auto sync = [&]() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  };
+  const double2* fra = lds_a + kq * S::LA + wm * (16 * SI) + l16;
+  const double2* frb = lds_b + kq * S::LB + wn * (16 * SJ) + l16;
+  auto read = [&](int fbuf, int buf, int ks) {
+#pragma unroll
+    for (int i = 0; i < SI; ++i) fa[fbuf][i] = fra[buf * (TK * S::LA) + ks * 4 * S::LA + 16 * i];
+#pragma unroll
+    for (int j = 0; j < SJ; ++j) fb[fbuf][j] = frb[buf * (TK * S::LB) + ks * 4 * S::LB + 16 * j];
+  };
+  double sgn_a = 1.0, sgn_b = 1.0;  // -1: the operand is conjugated
+  auto mma = [&](int f) {
+    if constexpr (k4M) {
+#pragma unroll
+      for (int i = 0; i < SI; ++i)
+#pragma unroll
+        for (int j = 0; j < SJ; ++j) {
+          acc1[i][j] = mfma(fa[f][i].x, fb[f][j].x, acc1[i][j]);
+          acc2[i][j] = mfma(fa[f][i].x, fb[f][j].y, acc2[i][j]);
+          acc1[i][j] = mfma_nega(fa[f][i].y, fb[f][j].y, acc1[i][j]);
+          acc2[i][j] = mfma(fa[f][i].y, fb[f][j].x, acc2[i][j]);
+        }
+      return;
+    }
+    double sa[SI], sb[SJ];
+#pragma unroll
+    for (int i = 0; i < SI; ++i)
+#pragma unroll
+      for (int j = 0; j < SJ; ++j) acc1[i][j] = mfma(fa[f][i].x, fb[f][j].x, acc1[i][j]);
+#pragma unroll
+    for (int i = 0; i < SI; ++i)
+#pragma unroll
+      for (int j = 0; j < SJ; ++j) acc2[i][j] = mfma(fa[f][i].y, fb[f][j].y, acc2[i][j]);
+#pragma unroll
+    for (int i = 0; i < SI; ++i) sa[i] = fma(sgn_a, fa[f][i].y, fa[f][i].x);
+#pragma unroll
+    for (int j = 0; j < SJ; ++j) sb[j] = fma(sgn_b, fb[f][j].y, fb[f][j].x);
+#pragma unroll
+    for (int i = 0; i < SI; ++i)
+#pragma unroll
+      for (int j = 0; j < SJ; ++j) acc3[i][j] = mfma(sa[i], sb[j], acc3[i][j]);
+  };
+
+  // acc1 and acc3 hold (neg1 ? -1 : 1) times the sum over the terms so far, acc2 (neg2 ? -1 : 1) times it
+  bool neg1 = false, neg2 = false;
+  for (int ti = 0; ti < P.nterms; ++ti) {
+    const ZTerm& T = P.t[ti];
+    const bool aN = T.opA == kOpN, bN = T.opB == kOpN;
+    const int K = T.k, lda = T.lda, ldb = T.ldb;
+    const int nt = (K + TK - 1) / TK;
+    if (nt == 0) continue;
+    const auto rsa = buf_of(T.A + (int64_t)e * T.sA), rsb = buf_of(T.B + (int64_t)e * T.sB);
+    const unsigned step_a = 16u * TK * (aN ? 1 : lda), step_b = 16u * TK * (bN ? ldb : 1);
+    unsigned offa[S::kAPer], offb[S::kBPer];
+    int ka[S::kAPer], kb[S::kBPer];
+#pragma unroll
+    for (int i = 0; i < S::kAPer; ++i) {
+      const int idx = tid + i * S::kThreads;
+      const int gm = m0 + (aN ? idx / TK : idx % TM);
+      ka[i] = aN ? idx % TK : idx / TM;
+      offa[i] = gm < m ? 16u * (aN ? gm * lda + ka[i] : ka[i] * lda + gm) : kOob;
+    }
+#pragma unroll
+    for (int i = 0; i < S::kBPer; ++i) {
+      const int idx = tid + i * S::kThreads;
+      const int gn = n0 + (bN ? idx % TN : idx / TK);
+      kb[i] = bN ? idx / TN : idx % TK;
+      offb[i] = gn < n ? 16u * (bN ? kb[i] * ldb + gn : gn * ldb + kb[i]) : kOob;
+    }
+    const double2 alpha = T.alpha;
+    {
+      const bool t1 = !kGen && alpha.x < 0.0, t2 = t1 != (aN != bN);
+      if (ti > 0 && t1 != neg1) {
+#pragma unroll
+        for (int i = 0; i < SI; ++i)
+#pragma unroll
+          for (int j = 0; j < SJ; ++j) {
+            acc1[i][j] = -acc1[i][j];
+            acc3[i][j] = -acc3[i][j];
+          }
+      }
+      if (ti > 0 && t2 != neg2) {
+#pragma unroll
+        for (int i = 0; i < SI; ++i)
+#pragma unroll
+          for (int j = 0; j < SJ; ++j) acc2[i][j] = -acc2[i][j];
+      }
+      neg1 = t1;
+      neg2 = t2;
+      sgn_a = aN ? 1.0 : -1.0;
+      sgn_b = bN ? 1.0 : -1.0;
+    }
+    double2* wa[S::kAPer];
+#pragma unroll
+    for (int i = 0; i < S::kAPer; ++i) {
+      const int idx = tid + i * S::kThreads;
+      wa[i] = lds_a + (aN ? (idx % TK) * S::LA + idx / TK : (idx / TM) * S::LA + idx % TM);
+    }
+    double2* wb[S::kBPer];
+#pragma unroll
+    for (int i = 0; i < S::kBPer; ++i) {
+      const int idx = tid + i * S::kThreads;
+      wb[i] = lds_b + (bN ? (idx / TN) * S::LB + idx % TN : (idx % TK) * S::LB + idx / TK);
+    }
+    auto load = [&](int t) {
+      t = min(t, nt - 1);
+      const int kr = K - t * TK;
+      const unsigned sa = t * step_a, sb = t * step_b;
+#pragma unroll
+      for (int i = 0; i < S::kAPer; ++i) ra[i] = buf_load(rsa, !kTail || ka[i] < kr ? offa[i] : kOob, sa);
+#pragma unroll
+      for (int i = 0; i < S::kBPer; ++i) rb[i] = buf_load(rsb, !kTail || kb[i] < kr ? offb[i] : kOob, sb);
+    };
+    auto store = [&](int buf) {
+#pragma unroll
+      for (int i = 0; i < S::kAPer; ++i) {
+        // (conjugate(a) alpha = conjugate(a conjugate(alpha)): the MFMAs conjugate)
+        wa[i][buf * (TK * S::LA)] = kGen ? cmul(aN ? alpha : cconj(alpha), ra[i]) : ra[i];
+      }
+#pragma unroll
+      for (int i = 0; i < S::kBPer; ++i) wb[i][buf * (TK * S::LB)] = rb[i];
+    };
+    load(0);
+    store(0);
+    load(1);
+    sync();
+    // One k-tile in LDS stage `cur`; the tile after the last one is loaded and
+    // stored again in its place, so that the loop has no condition.
+    auto tile = [&](int t, int cur) {
+      constexpr int kM = (k4M ? 4 : 3) * SI * SJ, kMem = S::kAPer + S::kBPer;
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (kLive) read(1, cur, 1);
+      store(cur ^ 1);
+      load(t + 2);
+      if constexpr (kLive) {
+        mma(0);
+#pragma unroll
+        for (int i = 0; i < SI + SJ; ++i) { QX_SGB(kSgMfma, 1); QX_SGB(kSgDsRead, 1); }
+#pragma unroll
+        for (int i = 0; i < kMem; ++i) { QX_SGB(kSgMfma, 1); QX_SGB(kSgDsWrite, 1); QX_SGB(kSgVmemRead, 1); }
+        QX_SGB(kSgMfma, kM);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      sync();
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (kLive) {
+        read(0, cur ^ 1, 0);
+        mma(1);
+#pragma unroll
+        for (int i = 0; i < SI + SJ; ++i) { QX_SGB(kSgMfma, 1); QX_SGB(kSgDsRead, 1); }
+        QX_SGB(kSgMfma, kM);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    if constexpr (kLive) read(0, 0, 0);
+#pragma unroll 1
+    for (int t = 0; t < nt; t += 2) {
+      tile(t, 0);
+      if (t + 1 == nt) break;
+      tile(t + 1, 1);
+    }
+    // every wave has read this term's last tile before the barrier in its
+    // middle; what the last store and read touched is not used
+    if (ti + 1 < P.nterms) sync();
+  }
+
+  // ---- epilogue, straight from the accumulators ----
+  if constexpr (!kLive) return;
+  const int64_t eo = e;
+  const auto rd = buf_of(P.D + eo * P.sD);
+  const auto rd2 = buf_of(P.D2 ? P.D2 + eo * P.sD2 : P.D);
+#pragma unroll
+  for (int i = 0; i < SI; ++i) {
+#pragma unroll
+    for (int j = 0; j < SJ; ++j) {
+      __builtin_amdgcn_sched_barrier(0);
+      const int col = nw + 16 * j + l16, row0 = mw + 16 * i + kq;
+      const int rows = col < n ? m : 0;  // rows of this column that are valid
+      auto at = [&](int ld, int r) { return row0 + 4 * r < rows ? 16u * ((row0 + 4 * r) * ld + col) : kOob; };
+      auto at_t = [&](int ld, int r) { return row0 + 4 * r < rows ? 16u * (col * ld + row0 + 4 * r) : kOob; };
+      double2 v[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const double p1 = neg1 ? -acc1[i][j][r] : acc1[i][j][r], p2 = neg2 ? -acc2[i][j][r] : acc2[i][j][r];
+        const double p3 = neg1 ? -acc3[i][j][r] : acc3[i][j][r];
+        v[r] = k4M ? cmk(p1, p2) : cmk(p1 - p2, p3 - p1 - p2);
+      }
+      for (int a = 0; a <= P.naddends; ++a) {
+        if (a == P.npre && P.d2mode == kD2Partial) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) buf_store(rd2, at(P.ldd2, r), v[r]);
+        }
+        if (a == P.naddends) break;
+        const ZAddend& A = P.ad[a];
+        const auto rf = buf_of(A.F + eo * A.sF);
+        if (cnz(A.c1)) {
+          double2 f[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) f[r] = buf_load(rf, at(A.ldf, r), 0);
+          if (cnz(A.c2)) {
+            double2 f2[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) f2[r] = buf_load(rf, at_t(A.ldf, r), 0);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = cadd(v[r], cadd(cmul(A.c1, f[r]), cmul(A.c2, cconj(f2[r]))));
+          } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = cadd(v[r], cmul(A.c1, f[r]));
+          }
+        } else if (cnz(A.c2)) {
+          double2 f2[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) f2[r] = buf_load(rf, at_t(A.ldf, r), 0);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[r] = cadd(v[r], cmul(A.c2, cconj(f2[r])));
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) buf_store(rd, at(P.ldd, r), v[r]);
+      if (P.d2mode == kD2Copy) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) buf_store(rd2, at(P.ldd2, r), cmul(P.s2, v[r]));
+      }
+      if (P.d2mode == kD2ConjT) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) buf_store(rd2, at_t(P.ldd2, r), cmul(P.s2, cconj(v[r])));
+      }
+    }
+  }
+  };
+  if (some) body(std::true_type{});
+  else body(std::false_type{});
+}
+
+template <int TM, int TN, int WM, int WN, int MINW, int kRole>
+hipError_t launch_3m(const ZGroup& g0, hipStream_t stream, bool plain4m = false) {
+  ZGroup g = g0;
+  int per = 0;
+  bool gen = false, tail = false;
+  for (int p = 0; p < g.nprob; ++p) {
+    const int tm = (g.p[p].m + TM - 1) / TM, tn = (g.p[p].n + TN - 1) / TN;
+    g.tiles_n[p] = tn;
+    g.tiles_mn[p] = tm * tn;
+    g.wg_base[p] = per;
+    per += tm * tn;
+    for (int t = 0; t < g.p[p].nterms; ++t) {
+      const ZTerm& T = g.p[p].t[t];
+      gen |= T.alpha.y != 0.0 || (T.alpha.x != 1.0 && T.alpha.x != -1.0);
+      tail |= T.k % Tile3M<TM, TN, WM, WN>::kTK != 0;
+    }
+  }
+  g.wg_base[g.nprob] = per;
+  const int64_t total = (int64_t)per * g.nE;
+  if (total == 0) return hipSuccess;
+  if (total > 0x7fffffff) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)total), block(64 * WM * WN);
+  if constexpr (kRole == 1 && TM == 32 && TN == 32) {
+    if (plain4m) {
+      hipLaunchKernelGGL((zgemm3m_kernel<TM, TN, WM, WN, MINW, kRole, kPlain4M>), grid, block, 0, stream, g);
+      return hipGetLastError();
+    }
+  }
+  if (gen) hipLaunchKernelGGL((zgemm3m_kernel<TM, TN, WM, WN, MINW, kRole, kGeneral>), grid, block, 0, stream, g);
+  else if (tail) hipLaunchKernelGGL((zgemm3m_kernel<TM, TN, WM, WN, MINW, kRole, kFastTail>), grid, block, 0, stream, g);
+  else hipLaunchKernelGGL((zgemm3m_kernel<TM, TN, WM, WN, MINW, kRole, kFast>), grid, block, 0, stream, g);
+  return hipGetLastError();
+}
+
+// The 3M tile of a launch: 64 x 64, 64 x 32 or 32 x 32, each by four waves.  A
+// larger tile reads less and spends fewer instructions per MFMA (relative
+// rates 1, 0.98 and 0.93 at 256^3 x 512), a smaller one wastes less at the edges and
+// in the last round over the 256 CUs: time ~ area (rounds + 1/2) / rate, with the
+// half round for a first load and an epilogue that nothing hides.  It
+// agrees with the fastest of the three at b = 64 ... 512, 8 ... 512 energies, to
+// 4% (us for 64 x 64 / 64 x 32 / 32 x 32: 3 products of 256^3 x 8 50.6 / 40.3 / 47.1,
+// 2 of 192^3 x 32 59.0 / 49.3 / 47.7, 4 of 208^3 x 64 318 / 278 / 254, 3 of
+// 512^3 x 16 549 / 561 / 593).  Products with K up to 64 (the inversion's trailing
+// updates) are bound by the latency of that first load, which three workgroups
+// per CU hide better than two: no 64 x 64 tile (256 x 192, K = 64, 512
+// energies: 307 / 257 / 263).
+int pick_3m(const ZGroup& g) {
+  const int tm[3] = {64, 64, 32}, tn[3] = {64, 32, 32};
+  const double rate[3] = {1.0, 0.978, 0.927};
+  int kmax = 0;
+  for (int p = 0; p < g.nprob; ++p) {
+    int k = 0;
+    for (int t = 0; t < g.p[p].nterms; ++t) k += g.p[p].t[t].k;
+    kmax = k > kmax ? k : kmax;
+  }
+  int best = 0;
+  double tbest = 0;
+  for (int c = kmax <= 64 ? 1 : 0; c < 3; ++c) {
+    int64_t wgs = 0;
+    for (int p = 0; p < g.nprob; ++p)
+      wgs += (int64_t)((g.p[p].m + tm[c] - 1) / tm[c]) * ((g.p[p].n + tn[c] - 1) / tn[c]);
+    wgs *= g.nE;
+    const double t = tm[c] * tn[c] * ((double)((wgs + 255) / 256) + 0.5) / rate[c];
+    if (tbest == 0 || t < tbest) {
+      best = c;
+      tbest = t;
+    }
+  }
+  return best;
+}
+
+template <int kRole>
+hipError_t launch_3m_auto(const ZGroup& g, hipStream_t stream) {
+  switch (pick_3m(g)) {
+    case 0: return launch_3m<64, 64, 2, 2, 2, kRole>(g, stream);
+    case 1: return launch_3m<64, 32, 2, 2, 3, kRole>(g, stream);
+    default: return launch_3m<32, 32, 2, 2, 4, kRole>(g, stream);
+  }
 }
 
 }  // namespace
@@ -471,9 +853,9 @@ hipError_t launch_zgemm(const ZGroup& g, int cfg, hipStream_t stream) {
     case kTile32x32: return launch_cfg<32, 32, 0>(g, stream);
     case kTile64x32: return launch_cfg<64, 32, 0>(g, stream);
     case kTile128x64: return launch_cfg<128, 64, 0>(g, stream);
-    case kTile64x64_3M: return launch_cfg<64, 64, 0, false, true>(g, stream);
-    case kTile32x32_3M: return launch_cfg<32, 32, 0, false, true>(g, stream);
-    case kTile128x64_3M: return launch_cfg<128, 64, 0, false, true, 16>(g, stream);
+    case kTile64x64_3M: return launch_3m_auto<0>(g, stream);
+    case kTile32x32_3M: return launch_3m<32, 32, 2, 2, 4, 0>(g, stream);
+    case kTile128x64_3M: return launch_3m<128, 64, 4, 2, 2, 0>(g, stream);
     default: return launch_cfg<64, 64, 0>(g, stream);
   }
 }
@@ -489,10 +871,13 @@ hipError_t launch_zgemm_f32(const ZGroup& g, int cfg, hipStream_t stream) {
 hipError_t launch_zgemm_update(const ZGroup& g, int cfg, hipStream_t stream) {
   switch (cfg) {
     case kTile32x32: return launch_cfg<32, 32, 1>(g, stream);
-    case kTile32x32_3M: return launch_cfg<32, 32, 1, false, true>(g, stream);
-    case kTile64x64_3M: case kTile128x64_3M: return launch_cfg<64, 64, 1, false, true>(g, stream);
+    case kTile32x32_3M: case kTile64x64_3M: case kTile128x64_3M: return launch_3m_auto<1>(g, stream);
     default: return launch_cfg<64, 64, 1>(g, stream);
   }
+}
+
+hipError_t launch_zgemm_narrow(const ZGroup& g, hipStream_t stream) {
+  return launch_3m<32, 32, 2, 2, 4, 1>(g, stream, true);
 }
 
 }  // namespace qx

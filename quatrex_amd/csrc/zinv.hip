@@ -598,10 +598,10 @@ hipError_t zinv_run(double2* S, int64_t sS, int n, int nE, double2* Out, int64_t
   };
   auto run = [&](ZGroup& g) { return g.nprob ? launch_zgemm_update(g, tile_cfg, stream) : hipSuccess; };
   // the narrow K = NB updates of a pair's panel columns on full 32 x 32 tiles
-  // (a 64 x 64 tile would be half empty; 512 inverses of 256 x 256: 3.16 ->
-  // 3.03 ms, the 3M 32 x 32 tile 3.10 ms)
+  // (a 64 x 64 tile would be half empty), four waves of 16 x 16 each (256 x 32,
+  // K = 32, 64 energies: 7.0 us, one wave of 32 x 32 15.0; 512 energies 37 / 40)
   auto run_narrow = [&](ZGroup& g) {
-    return g.nprob ? launch_zgemm_update(g, kTile32x32, stream) : hipSuccess;
+    return g.nprob ? launch_zgemm_narrow(g, stream) : hipSuccess;
   };
   hipError_t err = hipSuccess;
   for (int k = 0; k < n;) {
