@@ -61,6 +61,20 @@ static __device__ inline double readlane_d(double x, int src) {
   return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
+// Buffer accesses: a 32-bit byte offset per lane and a scalar offset; an offset of
+// kOob lies beyond every buffer, where loads give zero and stores are dropped.
+typedef unsigned uint4_t __attribute__((ext_vector_type(4)));
+constexpr unsigned kOob = 0x80000000u;
+__device__ inline __amdgpu_buffer_rsrc_t buf_of(const void* p) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, 0x7fffffff, 0x00020000);
+}
+__device__ inline double2 buf_load(__amdgpu_buffer_rsrc_t r, unsigned off, unsigned soff) {
+  return __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(r, off, soff, 0));
+}
+__device__ inline void buf_store(__amdgpu_buffer_rsrc_t r, unsigned off, double2 v) {
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4_t, v), r, off, 0, 0);
+}
+
 enum Op : int32_t { kOpN = 0, kOpC = 1 };
 enum D2Mode : int32_t { kD2None = 0, kD2Partial = 1, kD2Copy = 2, kD2ConjT = 3 };
 

@@ -444,18 +444,6 @@ hipError_t launch_cfg(const ZGroup& g0, hipStream_t stream) {
 #define QX_SGB(mask, n) __builtin_amdgcn_sched_group_barrier(mask, n, 0)
 constexpr int kSgMfma = 0x8, kSgVmemRead = 0x20, kSgDsRead = 0x100, kSgDsWrite = 0x200;
 
-typedef unsigned uint4_t __attribute__((ext_vector_type(4)));
-constexpr unsigned kOob = 0x80000000u;  // beyond num_records: loads give 0, stores are dropped
-__device__ inline __amdgpu_buffer_rsrc_t buf_of(const void* p) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, 0x7fffffff, 0x00020000);
-}
-__device__ inline double2 buf_load(__amdgpu_buffer_rsrc_t r, unsigned off, unsigned soff) {
-  return __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(r, off, soff, 0));
-}
-__device__ inline void buf_store(__amdgpu_buffer_rsrc_t r, unsigned off, double2 v) {
-  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4_t, v), r, off, 0, 0);
-}
-
 // kFast: alpha = +-1, every K a multiple of 8; kFastTail: alpha = +-1;
 // kGeneral: any.  kPlain4M: four MFMAs per product (no conjugation, alpha = 1).
 enum Form : int { kFast = 0, kFastTail = 1, kGeneral = 2, kPlain4M = 3 };

@@ -5,10 +5,11 @@
 // |re|+|im| among the rows not yet used as pivots (LAPACK izamax's measure,
 // first physical row on ties).  Nothing is swapped: after all steps the matrix
 // holds M with A^{-1}[i][j] = M[pi(i)][pi^{-1}(j)].  A panel of NB columns
-// [k, k+nb) is eliminated by zinv_panel_kernel (one workgroup per energy, one
-// physical row per thread, the row's panel part in registers; for matrices up
-// to 32 rows zinv_panel2_kernel, two threads per row): unblocked GJE on the
-// panel.  In zinv_panel_kernel a step takes one barrier: before it every
+// [k, k+nb) is eliminated by a panel kernel, one workgroup per energy and
+// unblocked GJE on the panel: zinv_panel2_kernel up to 32 rows (two threads per
+// row), zinv_panel8_kernel up to 512 (sub-panels of 8 columns), zinv_panel_kernel above
+// (16-column panels, one physical row per thread with its panel part in
+// registers).  In zinv_panel_kernel a step takes one barrier: before it every
 // wave publishes its best candidate row (DPP maximum of the key) and the
 // key; after it every thread takes the winner and applies
 //   row <- keep row + g prow   (keep = 1, g = -a_r / a_p; for the pivot row
@@ -83,6 +84,33 @@ __device__ inline double row_max16_d(double v) {
   v = fmax(v, dpp_d<0x114>(v));
   v = fmax(v, dpp_d<0x118>(v));
   return v;
+}
+
+__device__ inline unsigned row_max16_u(unsigned v) {
+  // (a lane whose source lies before its row takes 0)
+  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, true));
+  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, true));
+  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, true));
+  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, true));
+  return v;
+}
+// 1 / d = conj(d) / |d|^2 without a branch: d scaled by a power of two to
+// max(|re|, |im|) in [1/2, 1), the reciprocal of |d|^2 by v_rcp_f64 and two
+// Newton steps, and the same power of two on the result.
+__device__ inline double2 scaled_recip(double2 d) {
+  const int ex = __builtin_amdgcn_frexp_exp(fmax(fabs(d.x), fabs(d.y)));
+  const double x = __builtin_amdgcn_ldexp(d.x, -ex), y = __builtin_amdgcn_ldexp(d.y, -ex);
+  const double m = x * x + y * y;
+  double r = __builtin_amdgcn_rcp(m);
+  r = fma(r, fma(-m, r, 1.0), r);
+  r = fma(r, fma(-m, r, 1.0), r);
+  return cmk(__builtin_amdgcn_ldexp(x * r, -ex), __builtin_amdgcn_ldexp(-y * r, -ex));
+}
+// Maximum of two wave-uniform values, on the scalar unit.
+__device__ inline unsigned max_uniform(unsigned a, unsigned b) {
+  unsigned r;
+  asm("s_max_u32 %0, %1, %2" : "=s"(r) : "s"(a), "s"(b) : "scc");
+  return r;
 }
 
 // Shared state of one panel workgroup.
@@ -321,6 +349,312 @@ zinv_panel_kernel(double2* S, int64_t sS, int n, int k, int nbe, char* aux, int6
       }
     }
   }
+}
+
+// The panel kernel of 33 to 512 rows: 32 columns in four sub-panels of 8.
+//
+// A step of the elimination is a chain (update the next pivot column, find its
+// largest unused entry, publish that row, read it back, scale), and the kernel is bound
+// by the length of that chain times n steps: at 4.1 cycles per FP64
+// instruction of a wave, 8.5 between dependent ones, 60 per LDS read and 25-55 per
+// 16-byte LDS write of a single lane.  So the unblocked elimination runs on 8
+// columns, one physical row per thread with its 8 values in registers (7 complex updates
+// and 8 published values per step instead of 31 and 32), and the panel's other 24 columns
+// follow once per sub-panel on the matrix cores: X += T W, with T the n x 8
+// result and W the 8 pivot rows of X (moved out of X, which keeps zeros there; the same
+// block step as between panels).  The panel itself stays in registers in the MFMA
+// accumulator layout, a wave's 64 rows as 4 x 2 tiles of 16 x 16, and a sub-panel passes
+// through the wave's own LDS area into the row layout and back, without a barrier.
+//  * pivot key: high word of |re| + |im| with the row in its low bits (10 of its 20
+//    mantissa bits decide, the first row on ties), so that a wave's maximum is four
+//    32-bit DPP steps and one word says key, row and wave;
+//  * two barriers per step: the waves' keys before the first, and only the winning row
+//    is written, before the second (one lane's 8 writes: 264 cycles, by four waves at
+//    once 468);
+//  * every lane forms the reciprocal of its own value beside the search, so the pivot's
+//    is there when its row wins; the pivot row starts from zero (its registers are
+//    cleared while the published row is on its way), so an update is four FMAs;
+//  * the panel is read and written in 256-byte row segments, all loads in flight,
+//    and the pivot rows' columns outside the panel move to Wp under the MFMAs.
+// Measured (MI355X, per launch, against one row of 32 columns per thread before): 128 and
+// 256 rows, 8 matrices 39.7 us (68), 512 rows, 16 matrices 58 (138), 512 matrices of 256
+// rows 82 (131).  Of the 39.7 us the 32 steps take about 19 (some 1400 cycles each), the 256 MFMAs
+// of a wave 7, their operands' way through LDS and the pivot rows 8, panel I/O 3.
+// Sub-panels of 16 (half the MFMAs, twice the published values) took 47 us, of 16 with
+// four lanes per row 57.
+constexpr int kSub = 8;
+constexpr int kWaveElems = 64 * 9;  // one wave's LDS area (row-major or k-major)
+
+// MW: at most this many waves.
+template <int MW>
+__global__ void __launch_bounds__(64 * MW, 2)
+zinv_panel8_kernel(double2* S, int64_t sS, int n, int k, int nbe, char* aux, int64_t sAux,
+                   int wp_slot, int* info, int info_tag, int64_t e0) {
+  constexpr int NB = 32;
+  constexpr unsigned kRow = 511u;  // row bits of a pivot key
+  const int e = blockIdx.x;
+  double2* A = S + (int64_t)e * sS;
+  char* ax = aux + (int64_t)e * sAux;
+  double2* Wp = reinterpret_cast<double2*>(ax + PanelAux<NB>::wp(n, wp_slot));
+  int* piv = reinterpret_cast<int*>(ax + PanelAux<NB>::piv(n));
+  int* step_of = reinterpret_cast<int*>(ax + PanelAux<NB>::step(n));
+
+  // the step's pivot row (with the reciprocal of the pivot in its place), and by
+  // step parity the key of each wave's best row (0: no unused row left)
+  __shared__ double2 cand[kSub];
+  __shared__ __align__(16) unsigned ckey[2][(MW + 3) & ~3];
+  __shared__ double2 W[kSub][NB];
+  __shared__ int s_piv[NB];
+  extern __shared__ __align__(16) double2 wave_area[];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nw = blockDim.x >> 6;
+  const int l16 = lane & 15, kq = lane >> 4;
+  const int row = tid, row0 = wave * 64;
+  const bool valid = row < n;
+  double2* T = wave_area + wave * kWaveElems;
+  if (tid < ((MW + 3) & ~3) && tid >= nw) ckey[0][tid] = ckey[1][tid] = 0u;
+  // step at which the row was the pivot (-1: unused; rows beyond the matrix count as used)
+  int step = valid ? (k > 0 ? step_of[row] : -1) : 0x7fffffff;
+
+  // the panel, zero beyond its rows and columns; register r of tile (rt, ct)
+  // is row 16 rt + 4 r + lane / 16 of the wave, column 16 ct + lane % 16
+  const auto rs = buf_of(A);
+  auto off = [&](int rt, int ct, int r, int kq_, int l16_) {
+    const int rr = row0 + rt * 16 + 4 * r + kq_, cc = ct * 16 + l16_;
+    return rr < n && cc < nbe ? 16u * (rr * n + k + cc) : kOob;
+  };
+  double4_t ar[4][2], ai[4][2];
+#pragma unroll
+  for (int ct = 0; ct < 2; ++ct)
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const double2 v = buf_load(rs, off(rt, ct, r, kq, l16), 0);
+        ar[rt][ct][r] = v.x;
+        ai[rt][ct][r] = v.y;
+      }
+  // LDS accesses of one wave are in order; this keeps the compiler from moving them
+  auto wave_fence = [&]() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+
+#pragma unroll
+  for (int ct = 0; ct < 2; ++ct) {
+#pragma unroll 1
+    for (int h = 0; h < 2; ++h) {
+      const int c0 = ct * 16 + h * 8;  // first column of the sub-panel
+      if (c0 >= nbe) break;
+      const int steps = min(kSub, nbe - c0);
+      const bool own = (l16 >> 3) == h;  // this lane's column of tile ct belongs to it
+      if (own) {
+#pragma unroll
+        for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            T[(rt * 16 + 4 * r + kq) * 9 + (l16 & 7)] = cmk(ar[rt][ct][r], ai[rt][ct][r]);
+      }
+      wave_fence();
+      // the row's 8 values, rotated by one position after every step: the
+      // current pivot column is always position 0 and the step loop stays rolled
+      double re[kSub], im[kSub];
+#pragma unroll
+      for (int q = 0; q < kSub; ++q) {
+        const double2 v = T[lane * 9 + q];
+        re[q] = v.x;
+        im[q] = v.y;
+      }
+      int sub = -1;  // this row's step within the sub-panel
+      unsigned kw = 0;
+      int cl = 0;
+      double2 inv = cmk(0.0, 0.0);
+      // the wave's candidate for the column of values (x, y): its key kw, lane cl and
+      // reciprocal
+      auto search = [&](double x, double y) {
+        const unsigned hi = (unsigned)(__double_as_longlong(fabs(x) + fabs(y)) >> 32);
+        unsigned key = (hi & ~(2 * kRow + 1)) | (kRow + 1) | (kRow - row);
+        key = row_max16_u(step < 0 ? key : 0u);
+        kw = max_uniform(max_uniform((unsigned)__builtin_amdgcn_readlane((int)key, 15),
+                                     (unsigned)__builtin_amdgcn_readlane((int)key, 31)),
+                         max_uniform((unsigned)__builtin_amdgcn_readlane((int)key, 47),
+                                     (unsigned)__builtin_amdgcn_readlane((int)key, 63)));
+        cl = (int)(kRow - (kw & kRow)) & 63;
+        // (every lane that of its own value, beside the search and the row update; the
+        // empty asm keeps it from being sunk into the publishing lane's branch)
+        inv = scaled_recip(cmk(x, y));
+        asm volatile("" : "+v"(inv.x), "+v"(inv.y));
+      };
+      search(re[0], im[0]);
+      if (lane == 0) ckey[0][wave] = kw;
+#pragma unroll 1
+      for (int j = 0; j < kSub; ++j) {
+        const int b = j & 1;
+        __syncthreads();
+        if (j >= steps) {  // beyond the panel: rotate only
+          const double r0 = re[0], i0 = im[0];
+#pragma unroll
+          for (int q = 1; q < kSub; ++q) {
+            re[q - 1] = re[q];
+            im[q - 1] = im[q];
+          }
+          re[kSub - 1] = r0;
+          im[kSub - 1] = i0;
+          continue;
+        }
+        unsigned km = 0;
+        if constexpr (MW <= 2) {
+          km = max(ckey[b][0], MW > 1 ? ckey[b][1] : 0u);
+        } else {
+#pragma unroll
+          for (int w = 0; w < MW; w += 4) {
+            const uint4 kk = *reinterpret_cast<const uint4*>(&ckey[b][w]);
+            km = max(max(km, max(kk.x, kk.y)), max(kk.z, kk.w));
+          }
+        }
+        km = (unsigned)__builtin_amdgcn_readfirstlane((int)km);
+        const int p = min((int)(kRow - (km & kRow)), n - 1);  // (the bound is for memory safety only)
+        if (row == p) {
+          cand[0] = inv;
+#pragma unroll
+          for (int q = 1; q < kSub; ++q) cand[q] = cmk(re[q], im[q]);
+        }
+        // The update is new[q - 1] = row[q] + g prow[q], new[last] = g with
+        // g = -a_r / a_p; the pivot row has g = 1 / a_p and starts from zero (while
+        // the published row is on its way)
+        const bool me = row == p;
+        const double a_re = re[0], a_im = im[0];
+        if (me) {
+          step = k + c0 + j;
+          sub = j;
+          s_piv[c0 + j] = p;
+          if (a_re == 0.0 && a_im == 0.0 && atomicCAS(info, 0, info_tag) == 0) {
+            info[1] = (int)(e0 + e);
+            info[2] = step;
+          }
+#pragma unroll
+          for (int q = 1; q < kSub; ++q) re[q] = im[q] = 0.0;
+        }
+        __syncthreads();
+        double2 pv[kSub];
+#pragma unroll
+        for (int q = 0; q < kSub; ++q) pv[q] = cand[q];
+        const double2 iv = pv[0];
+        const double gr = me ? iv.x : -(a_re * iv.x - a_im * iv.y);
+        const double gi = me ? iv.y : -(a_re * iv.y + a_im * iv.x);
+        auto upd = [&](int q) {
+          re[q - 1] = fma(gr, pv[q].x, fma(-gi, pv[q].y, re[q]));
+          im[q - 1] = fma(gr, pv[q].y, fma(gi, pv[q].x, im[q]));
+        };
+        upd(1);
+        search(re[0], im[0]);  // (after the last step: of a finished column, not used)
+        if (lane == 0) ckey[b ^ 1][wave] = kw;
+#pragma unroll
+        for (int q = 2; q < kSub; ++q) upd(q);
+        re[kSub - 1] = gr;
+        im[kSub - 1] = gi;
+      }
+      // T, k-major, for the MFMAs and the way back into the tile
+      wave_fence();
+#pragma unroll
+      for (int q = 0; q < kSub; ++q) T[q * 65 + lane] = cmk(re[q], im[q]);
+      // the pivot rows leave the panel and leave zeros
+      const unsigned long long chosen = __ballot(sub >= 0);
+#pragma unroll
+      for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int base = rt * 16 + 4 * r;
+          if (((chosen >> base) & 15) == 0) continue;
+          const int s0 = __builtin_amdgcn_readlane(sub, base), s1 = __builtin_amdgcn_readlane(sub, base + 1);
+          const int s2 = __builtin_amdgcn_readlane(sub, base + 2), s3 = __builtin_amdgcn_readlane(sub, base + 3);
+          const int ps = kq == 0 ? s0 : kq == 1 ? s1 : kq == 2 ? s2 : s3;
+          if (ps >= 0) {
+#pragma unroll
+            for (int t2 = 0; t2 < 2; ++t2) {
+              W[ps][t2 * 16 + l16] = cmk(ar[rt][t2][r], ai[rt][t2][r]);
+              ar[rt][t2][r] = 0.0;
+              ai[rt][t2][r] = 0.0;
+            }
+          }
+        }
+      __syncthreads();
+      double2 bw[2][2], a[4][2];
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int t2 = 0; t2 < 2; ++t2) {
+          bw[ks][t2] = W[ks * 4 + kq][t2 * 16 + l16];
+          if (ks * 4 + kq >= steps || (t2 == ct && own)) bw[ks][t2] = cmk(0.0, 0.0);
+        }
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int rt = 0; rt < 4; ++rt) a[rt][ks] = T[(ks * 4 + kq) * 65 + rt * 16 + l16];
+      auto mul = [&](int ks) {
+#pragma unroll
+        for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+          for (int t2 = 0; t2 < 2; ++t2) {
+            ar[rt][t2] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[rt][ks].x, bw[ks][t2].x, ar[rt][t2], 0, 0, 0);
+            ai[rt][t2] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[rt][ks].x, bw[ks][t2].y, ai[rt][t2], 0, 0, 0);
+            ar[rt][t2] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[rt][ks].y, bw[ks][t2].y, ar[rt][t2], 0, 0, 1);
+            ai[rt][t2] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[rt][ks].y, bw[ks][t2].x, ai[rt][t2], 0, 0, 0);
+          }
+      };
+      mul(0);
+      __builtin_amdgcn_sched_barrier(0);
+      // the pivot rows' columns outside the panel, one column per thread: loaded
+      // and, after the other half of the MFMAs, stored
+      const bool outside = tid < n && (tid < k || tid >= k + nbe);
+      int pr[kSub];
+      double2 mv[kSub];
+#pragma unroll
+      for (int q = 0; q < kSub; ++q) pr[q] = s_piv[c0 + q];
+#pragma unroll
+      for (int q = 0; q < kSub; ++q)
+        mv[q] = buf_load(rs, outside && q < steps ? 16u * (pr[q] * n + tid) : kOob, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      mul(1);
+      __builtin_amdgcn_sched_barrier(0);
+      // the sub-panel's columns come back into the tile
+      {
+        double2 v[16];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) v[q] = T[(l16 & 7) * 65 + 4 * q + kq];
+#pragma unroll
+        for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            ar[rt][ct][r] = own ? v[4 * rt + r].x : ar[rt][ct][r];
+            ai[rt][ct][r] = own ? v[4 * rt + r].y : ai[rt][ct][r];
+          }
+      }
+      if (outside) {
+#pragma unroll
+        for (int q = 0; q < kSub; ++q)
+          if (q < steps) {
+            Wp[(int64_t)(c0 + q) * n + tid] = mv[q];
+            A[(int64_t)pr[q] * n + tid] = cmk(0.0, 0.0);
+          }
+      }
+      wave_fence();
+    }
+  }
+  if (valid) step_of[row] = step;
+  if (tid < nbe) piv[k + tid] = s_piv[tid];
+  // (the offsets are formed again instead of living through the kernel)
+  int kq2 = kq, l2 = l16;
+  asm volatile("" : "+v"(kq2), "+v"(l2));
+#pragma unroll
+  for (int ct = 0; ct < 2; ++ct)
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        buf_store(rs, off(rt, ct, r, kq2, l2), cmk(ar[rt][ct][r], ai[rt][ct][r]));
 }
 
 // The same elimination with two threads per row for 32-column panels: lanes l and l + 32 of a wave hold the two 16-column halves of
@@ -564,23 +898,23 @@ hipError_t zinv_run(double2* S, int64_t sS, int n, int nE, double2* Out, int64_t
   double2* wb = reinterpret_cast<double2*>(ax + PanelAux<NB>::wp(n, 1));
   // blocks up to 32: two threads per row, which fills the wave that one thread
   // per row would leave half idle (measured at 4096 matrices of 32 x 32: 0.196
-  // against 0.275 ms).  Larger blocks keep one thread per row: with two, a
-  // 256-row panel needs 8 waves of 152 VGPRs and one workgroup fills a CU
-  // (3.92 against 3.50 ms for 512 matrices of 256 x 256).
+  // against 0.275 ms)
   const bool two = NB == 32 && n <= 32;
   const int threads = two ? 2 * ((n + 31) / 32) * 32 : ((n + 63) / 64) * 64;
   auto panel = [&](int k, int nbe, int slot) {
+    auto go = [&](auto kern, size_t lds) {
+      hipLaunchKernelGGL(kern, dim3(nE), dim3(threads), lds, stream, S, sS, n, k, nbe, ax, sAux, slot, info,
+                         info_tag, e0);
+    };
     if constexpr (NB == 32) {
-      if (two) {
-        hipLaunchKernelGGL((zinv_panel2_kernel<512>), dim3(nE), dim3(threads),
-                           panel_stage_bytes(threads / 2), stream, S, sS, n, k, nbe, ax, sAux,
-                           slot, info, info_tag, e0);
-        return;
-      }
+      const size_t lds = (size_t)(threads / 64) * kWaveElems * sizeof(double2);
+      if (two) go(zinv_panel2_kernel<512>, panel_stage_bytes(threads / 2));
+      else if (threads <= 128) go(zinv_panel8_kernel<2>, lds);
+      else if (threads <= 256) go(zinv_panel8_kernel<4>, lds);
+      else go(zinv_panel8_kernel<8>, lds);
+    } else {
+      go(zinv_panel_kernel<NB, MAXT>, panel_stage_bytes(threads));
     }
-    hipLaunchKernelGGL((zinv_panel_kernel<NB, MAXT>), dim3(nE), dim3(threads),
-                       panel_stage_bytes(threads), stream, S, sS, n, k, nbe, ax, sAux, slot, info,
-                       info_tag, e0);
   };
   // operands: columns c0.. of S (stride sS) or of a pivot-row buffer (stride sAuxC), ld n
   auto tS = [&](int c0, const double2* B, int k) {
