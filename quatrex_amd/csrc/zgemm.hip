@@ -435,12 +435,12 @@ hipError_t launch_cfg(const ZGroup& g0, hipStream_t stream) {
 // matrix only help to stage.
 // Measured (MI355X, TFLOP/s by 8 m n k, against the kernel it replaced, which
 // staged its epilogue through LDS, waited for its own LDS traffic and relied on
-// a third workgroup per CU): 256^3 x 512 energies 89 (76), 512^3 x 16 94 (76),
-// 256^3 x 8 80 (48), 208^3 x 64 73 (49), 96^3 x 64 67 (36), 91 x 77 x 65 x 48
-// 33 (17); results are bit for bit the same.  90% of the time the matrix cores
+// a third workgroup per CU): 256^3 x 512 energies 93 (76), 512^3 x 16 96 (76),
+// 256^3 x 8 81 (48), 208^3 x 64 74 (49), 96^3 x 64 69 (36), 91 x 77 x 65 x 48
+// 33 (17); results are bit for bit the same.  92% of the time the matrix cores
 // are busy at 512^3; the rest is the FP64 adds of the fragment sums (5%) and
-// the epilogue.  Two waves per SIMD at 64 x 64 (256 registers) beat three (168,
-// spilled: 76).
+// the epilogue.  Three waves per SIMD at 64 x 64 (162 registers) hide prologues
+// and epilogues that two did not (256^3 x 512: 89).
 #define QX_SGB(mask, n) __builtin_amdgcn_sched_group_barrier(mask, n, 0)
 constexpr int kSgMfma = 0x8, kSgVmemRead = 0x20, kSgDsRead = 0x100, kSgDsWrite = 0x200;
 
@@ -546,12 +546,12 @@ __global__ void __launch_bounds__(64 * WM * WN, MINW) zgemm3m_kernel(const ZGrou
 
   // acc1 and acc3 hold (neg1 ? -1 : 1) times the sum over the terms so far, acc2 (neg2 ? -1 : 1) times it
   bool neg1 = false, neg2 = false;
-  for (int ti = 0; ti < P.nterms; ++ti) {
+  auto term = [&](int ti) {
     const ZTerm& T = P.t[ti];
     const bool aN = T.opA == kOpN, bN = T.opB == kOpN;
     const int K = T.k, lda = T.lda, ldb = T.ldb;
     const int nt = (K + TK - 1) / TK;
-    if (nt == 0) continue;
+    if (nt == 0) return;
     const auto rsa = buf_of(T.A + (int64_t)e * T.sA), rsb = buf_of(T.B + (int64_t)e * T.sB);
     const unsigned step_a = 16u * TK * (aN ? 1 : lda), step_b = 16u * TK * (bN ? ldb : 1);
     unsigned offa[S::kAPer], offb[S::kBPer];
@@ -665,7 +665,12 @@ __global__ void __launch_bounds__(64 * WM * WN, MINW) zgemm3m_kernel(const ZGrou
     // every wave has read this term's last tile before the barrier in its
     // middle; what the last store and read touched is not used
     if (ti + 1 < P.nterms) sync();
-  }
+  };
+  // Written out, not a loop: round a loop the compiler keeps a second copy of
+  // every accumulator (64 x 64: 256 registers instead of 166).
+  static_assert(sizeof(P.t) / sizeof(P.t[0]) == 2, "a problem has up to two terms");
+  if (P.nterms > 0) term(0);
+  if (P.nterms > 1) term(1);
 
   // ---- epilogue, straight from the accumulators ----
   if constexpr (!kLive) return;
@@ -771,25 +776,26 @@ hipError_t launch_3m(const ZGroup& g0, hipStream_t stream, bool plain4m = false)
 
 // The 3M tile of a launch: 64 x 64, 64 x 32 or 32 x 32, each by four waves.  A
 // larger tile reads less and spends fewer instructions per MFMA (relative
-// rates 1, 0.98 and 0.93 at 256^3 x 512), a smaller one wastes less at the edges and
+// rates 1, 0.944 and 0.884 at 256^3 x 512), a smaller one wastes less at the edges and
 // in the last round over the 256 CUs: time ~ area (rounds + 1/2) / rate, with the
 // half round for a first load and an epilogue that nothing hides.  It
-// agrees with the fastest of the three at b = 64 ... 512, 8 ... 512 energies, to
-// 4% (us for 64 x 64 / 64 x 32 / 32 x 32: 3 products of 256^3 x 8 50.6 / 40.3 / 47.1,
-// 2 of 192^3 x 32 59.0 / 49.3 / 47.7, 4 of 208^3 x 64 318 / 278 / 254, 3 of
-// 512^3 x 16 549 / 561 / 593).  Products with K up to 64 (the inversion's trailing
-// updates) are bound by the latency of that first load, which three workgroups
-// per CU hide better than two: no 64 x 64 tile (256 x 192, K = 64, 512
-// energies: 307 / 257 / 263).
+// agrees with the fastest of the three at b = 48 ... 512, 8 ... 1024 energies, to
+// 4% (us for 64 x 64 / 64 x 32 / 32 x 32: 3 products of 256^3 x 8 49.6 / 39.8 / 40.6,
+// 2 of 192^3 x 32 55.6 / 48.5 / 47.0, 4 of 208^3 x 64 303 / 270 / 251, 3 of
+// 512^3 x 16 538 / 558 / 592).  Products with K up to 64 (small blocks and the inversion's
+// trailing updates) are bound by the latency of that first load and by the
+// epilogue, which more and smaller workgroups hide better: no 64 x 64 tile, and 32 x 32 as
+// fast per element as 64 x 32 (256 x 192, K = 64, 64 energies: 32.0 / 30.4 /
+// 30.0; 3 of 64^3 x 256 34.2 / 34.3 / 32.0; 3 of 48^3 x 1024 87 / 84 / 79).
 int pick_3m(const ZGroup& g) {
   const int tm[3] = {64, 64, 32}, tn[3] = {64, 32, 32};
-  const double rate[3] = {1.0, 0.978, 0.927};
   int kmax = 0;
   for (int p = 0; p < g.nprob; ++p) {
     int k = 0;
     for (int t = 0; t < g.p[p].nterms; ++t) k += g.p[p].t[t].k;
     kmax = k > kmax ? k : kmax;
   }
+  const double rate[3] = {1.0, 0.944, kmax <= 64 ? 0.935 : 0.884};
   int best = 0;
   double tbest = 0;
   for (int c = kmax <= 64 ? 1 : 0; c < 3; ++c) {
@@ -809,8 +815,8 @@ int pick_3m(const ZGroup& g) {
 template <int kRole>
 hipError_t launch_3m_auto(const ZGroup& g, hipStream_t stream) {
   switch (pick_3m(g)) {
-    case 0: return launch_3m<64, 64, 2, 2, 2, kRole>(g, stream);
-    case 1: return launch_3m<64, 32, 2, 2, 3, kRole>(g, stream);
+    case 0: return launch_3m<64, 64, 2, 2, 3, kRole>(g, stream);
+    case 1: return launch_3m<64, 32, 2, 2, 4, kRole>(g, stream);
     default: return launch_3m<32, 32, 2, 2, 4, kRole>(g, stream);
   }
 }
