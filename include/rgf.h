@@ -51,8 +51,8 @@ extern "C" {
                                       ungrouped op sequence; with RGF_OPT_MAX_CHUNK = 1 this is
                                       the one-energy-at-a-time baseline)                      */
 #define RGF_OPT_OVERLAP 6          /* 1 (default): each block inversion runs on a second stream of
-                                      default priority, overlapped with the independent
-                                      lesser/greater products of its forward step              */
+                                      default priority, beside the lesser and greater
+                                      products of its own and the previous block            */
 #define RGF_OPT_PROFILE 4          /* 1: time every sweep GEMM launch and every block inversion
                                       with HIP events on the context stream (0: off)          */
 #define RGF_OPT_PERSISTENT 7       /* 1 (default): FP64 selected solves of geometries whose blocks

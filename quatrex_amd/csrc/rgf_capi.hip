@@ -538,21 +538,52 @@ int sweep_chunk_solve(Ctx* c, const Geo& g, int64_t e0, int E, const SolveIO& io
   // ---- block 0 (rgf.py:216-239) ----
   {
     const int b = (int)g.bs[0];
-    Mat S = sl(0, b), Vl = sl(1, b), Vg = sl(2, b);
+    Mat S = sl(0, b);
     rc = c->gemm({PB(b, b).add(A.D(0), ONE).add(OR(0), MONE).out(S).done()}, E, b);
     if (rc) return rc;
     rc = c->inv(S.p, S.s, b, E, GR.D(0), w.aux, 1, e0);
     if (rc) return rc;
+  }
+  // V = g_j W ; g^<>_j = V g_j^H   (V shares the slots of Y).  Products that can
+  // run in V's launch go into `with`.
+  auto lesser_greater_0 = [&](const std::vector<ZProblem>& with) {
+    const int b = (int)g.bs[0];
+    Mat Vl = sl(4, b), Vg = sl(5, b);
     PB vl(b, b), vg(b, b);
     vl.term(GR.D(0), kOpN, SL.D(0), kOpN, b);
     vg.term(GR.D(0), kOpN, SG.D(0), kOpN, b);
     if (OL(0).p) vl.term(GR.D(0), kOpN, OL(0), kOpN, b);
     if (OG(0).p) vg.term(GR.D(0), kOpN, OG(0), kOpN, b);
-    rc = c->gemm({vl.out(Vl).done(), vg.out(Vg).done()}, E, b);
-    if (rc) return rc;
-    rc = c->gemm({PB(b, b).term(Vl, kOpN, GR.D(0), kOpC, b).out(GL.D(0)).done(),
-                  PB(b, b).term(Vg, kOpN, GR.D(0), kOpC, b).out(GG.D(0)).done()},
-                 E, b);
+    std::vector<ZProblem> l{vl.out(Vl).done(), vg.out(Vg).done()};
+    l.insert(l.end(), with.begin(), with.end());
+    int r = c->gemm(l, E, b);
+    if (r) return r;
+    return c->gemm({PB(b, b).term(Vl, kOpN, GR.D(0), kOpC, b).out(GL.D(0)).done(),
+                    PB(b, b).term(Vg, kOpN, GR.D(0), kOpC, b).out(GG.D(0)).done()},
+                   E, b);
+  };
+  auto lesser_greater = [&](int j, const std::vector<ZProblem>& with) {
+    if (j == 0) return lesser_greater_0(with);
+    const int bj = (int)g.bs[j];
+    Mat Wl = sl(6, bj), Wg = sl(7, bj), Vl = sl(4, bj), Vg = sl(5, bj);
+    std::vector<ZProblem> l{PB(bj, bj).term(GR.D(j), kOpN, Wl, kOpN, bj).out(Vl).done(),
+                            PB(bj, bj).term(GR.D(j), kOpN, Wg, kOpN, bj).out(Vg).done()};
+    l.insert(l.end(), with.begin(), with.end());
+    int r = c->gemm(l, E, bj);
+    if (r) return r;
+    return c->gemm({PB(bj, bj).term(Vl, kOpN, GR.D(j), kOpC, bj).out(GL.D(j)).done(),
+                    PB(bj, bj).term(Vg, kOpN, GR.D(j), kOpC, bj).out(GG.D(j)).done()},
+                   E, bj);
+  };
+  // With overlap the chain g_i -> P -> S -> g_j runs ahead: an inversion, which is bound
+  // by latency and leaves most CUs idle, has beside it (on the side stream) all ten lesser and
+  // greater products of a step, V and g^<> of block i, Q, Y and W, instead of the two W.
+  // The same products in another order (32 blocks of 256, 64 energies: 120.9 -> 116.1 ms, 16
+  // of 128 x 64 11.8 -> 11.0, 20 of 256 x 8, captured, 17.5 -> 16.7).  FP32 products keep
+  // the plain order: their Newton steps change g_j after the inversion.
+  const bool ahead = c->overlap && !c->prec32;
+  if (!ahead || N == 1) {
+    rc = lesser_greater(0, {});
     if (rc) return rc;
   }
 
@@ -573,7 +604,16 @@ int sweep_chunk_solve(Ctx* c, const Geo& g, int64_t e0, int E, const SolveIO& io
                             .done();
     const ZProblem pQl = PB(bj, bj).term(P, kOpN, SL.U(i), kOpN, bi).out(Ql).done();
     const ZProblem pQg = PB(bj, bj).term(P, kOpN, SG.U(i), kOpN, bi).out(Qg).done();
-    if (c->prec32 && c->refine < 0) {
+    const bool ovl = c->overlap;
+    if (ahead) {
+      rc = c->gemm({pP}, E, bj);
+      if (!rc) rc = c->gemm({pS}, E, bj);
+      if (!rc) rc = c->fork();
+      if (!rc) rc = c->inv(S.p, S.s, bj, E, GR.D(j), w.aux, j + 1, e0, c->side);
+      if (!rc) rc = lesser_greater(i, {pQl, pQg});
+      if (!rc) rc = c->gemm({pYl, pYg}, E, bj);
+      if (rc) return rc;
+    } else if (c->prec32 && c->refine < 0) {
       // Mixed precision with FP64 Schur complements: P and S in FP64, so the
       // inversion gets the exact FP64 S (the Newton steps' fixed point);
       // Y and Q stay FP32 products, in one launch after P.
@@ -593,8 +633,7 @@ int sweep_chunk_solve(Ctx* c, const Geo& g, int64_t e0, int E, const SolveIO& io
       if (rc) return rc;
     }
     // g_j = S^{-1} is independent of W: with overlap it runs on the side stream
-    const bool ovl = c->overlap;
-    if (ovl) {
+    if (ovl && !ahead) {
       rc = c->fork();
       if (rc) return rc;
       rc = c->inv(S.p, S.s, bj, E, GR.D(j), w.aux, j + 1, e0, c->side);
@@ -650,16 +689,10 @@ int sweep_chunk_solve(Ctx* c, const Geo& g, int64_t e0, int E, const SolveIO& io
       rc = c->gemm({PB(bj, bj).add(Gt, ONE).out(GR.D(j)).done()}, E, bj);
       if (rc) return rc;
     }
-    // V = g_j W ; g^<>_j = V g_j^H   (V reuses the Y slots)
-    Mat Vl = sl(4, bj), Vg = sl(5, bj);
-    rc = c->gemm({PB(bj, bj).term(GR.D(j), kOpN, Wl, kOpN, bj).out(Vl).done(),
-                  PB(bj, bj).term(GR.D(j), kOpN, Wg, kOpN, bj).out(Vg).done()},
-                 E, bj);
-    if (rc) return rc;
-    rc = c->gemm({PB(bj, bj).term(Vl, kOpN, GR.D(j), kOpC, bj).out(GL.D(j)).done(),
-                  PB(bj, bj).term(Vg, kOpN, GR.D(j), kOpC, bj).out(GG.D(j)).done()},
-                 E, bj);
-    if (rc) return rc;
+    if (!ahead || j == N - 1) {
+      rc = lesser_greater(j, {});
+      if (rc) return rc;
+    }
   }
 
   // ---- backward sweep (rgf.py:315-412) ----

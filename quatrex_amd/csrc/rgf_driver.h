@@ -78,8 +78,8 @@ struct Ctx {
   // sweep (one workgroup per energy, intermediates in LDS)
   bool persistent = true;
   int n_cu = 256;  // compute units of the device (persistent grid size)
-  // run each block inversion on a second stream, overlapped with the
-  // independent lesser/greater products of the same forward step
+  // run each block inversion on a second stream, beside the lesser and
+  // greater products that do not need it
   bool overlap = true;
   hipStream_t side = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;

@@ -462,6 +462,7 @@ struct Tile3M {
 // inside the blocked inversion.
 template <int TM, int TN, int WM, int WN, int MINW, int kRole, int kForm>
 __global__ void __launch_bounds__(64 * WM * WN, MINW) zgemm3m_kernel(const ZGroup g) {
+  if (kRole == 1) __builtin_amdgcn_s_setprio(2);  // the inversion is the longer chain
   using S = Tile3M<TM, TN, WM, WN>;
   constexpr int SI = S::SI, SJ = S::SJ, TK = S::kTK;
   constexpr bool kGen = kForm == kGeneral, kTail = kForm != kFast, k4M = kForm == kPlain4M;

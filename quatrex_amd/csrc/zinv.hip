@@ -390,6 +390,7 @@ template <int MW>
 __global__ void __launch_bounds__(64 * MW, 2)
 zinv_panel8_kernel(double2* S, int64_t sS, int n, int k, int nbe, char* aux, int64_t sAux,
                    int wp_slot, int* info, int info_tag, int64_t e0) {
+  __builtin_amdgcn_s_setprio(3);  // before the products that share its CU (+1% of a solve)
   constexpr int NB = 32;
   constexpr unsigned kRow = 511u;  // row bits of a pivot key
   const int e = blockIdx.x;
