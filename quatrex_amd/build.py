@@ -34,6 +34,12 @@ HIPCC_FLAGS = [
     "-munsafe-fp-atomics",
 ]
 
+# MFMA results in VGPRs also where a kernel has AGPRs to spare: the small sweep reads
+# every result back, and a copy costs an instruction per register (5% of a sweep).
+FILE_FLAGS = {
+    "sweep_small": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+}
+
 
 def hipcc() -> str:
     for cand in (os.environ.get("HIPCC"), shutil.which("hipcc"), "/opt/rocm/bin/hipcc"):
@@ -48,7 +54,7 @@ def sources() -> list[Path]:
 
 def _compile(src: Path, verbose: bool) -> Path:
     obj = OBJDIR / (src.stem + ".o")
-    cmd = [hipcc(), *HIPCC_FLAGS, "-I", str(CSRC), "-I", str(PKG.parent / "include"), "-c", str(src),
+    cmd = [hipcc(), *HIPCC_FLAGS, *FILE_FLAGS.get(src.stem, []), "-I", str(CSRC), "-I", str(PKG.parent / "include"), "-c", str(src),
            "-o", str(obj)]
     if verbose:
         print(" ".join(cmd), flush=True)

@@ -226,7 +226,7 @@ hipError_t launch_c2z(const float2* src, int64_t sSrc, double2* dst, int64_t sDs
 // retarded output is absent and the Sigma~ blocks of the current.
 constexpr int kSmallMaxBlock = 32;
 struct SmallProblem {
-  int32_t N, nE, job0, pad_;
+  int32_t N, nE, job0, full;  // full: every block above 16
   int64_t e_base, Dsz, Usz;
   const int* bs;
   const int64_t* od;

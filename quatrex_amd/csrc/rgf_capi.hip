@@ -902,6 +902,7 @@ int run_small(Ctx* c, std::vector<SmallSpec> specs, char* scratch) {
     q.N = g.N;
     q.nE = (int32_t)sp.nE;
     q.job0 = job0;
+    q.full = *std::min_element(bs.begin(), bs.end()) > 16;
     q.e_base = 0;
     q.Dsz = g.Dsz;
     q.Usz = g.Usz;

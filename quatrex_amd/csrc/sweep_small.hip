@@ -19,14 +19,30 @@
 // T1 = K g^<_i - B U^H term (the same products as the reference, grouped
 // to fit the nine slots).
 //
-// Products run in rounds: a round is a set of products that do not depend
-// on one another, wave w computes one 16 x 16 output tile of each of them
-// (tile (w - p) mod 4 of product p, so that products smaller than 16 x 16
-// spread over the waves), and the round ends with one barrier.  A round whose
-// outputs overwrite one of its own operands waits for every wave once more
-// before writing.  Outputs that are only stored (G^R_ij, G^R_ji, G_ii,
+// The forward sweep is bound by the inversions, one wave's serial pivot steps (39000
+// cycles for 32 x 32, of 100000 per block), so only P = A_ji g_i and S = A_jj - P A_ij stand
+// between two of them: while wave 3 inverts S, waves 0 and 1 run the lesser and greater
+// chains (V = g_i W_i, g^<>_i = V g_i^H, Y = A_ji g^<>_i, W_j; whole products by one
+// wave, in place, no barrier) and wave 2 forms their Q, stores g_i and brings
+// the next step's blocks.  Bytes are no limit (2.4 TB/s with 256 energies in flight).
+//
+// Elsewhere products run in rounds: a round is a set of products that do not depend
+// on one another, each wave computes one 16 x 16 output tile of each of them, and
+// the round ends with one barrier.  A round whose outputs overwrite one of its own operands
+// waits for every wave once more before writing.  With every block above 16 a
+// wave has the same tile in all products of a round and their common fragments are read once;
+// otherwise tile (w - p) mod 4 of product p, so that products smaller than 16 x 16
+// spread over the waves.  Outputs that are only stored (G^R_ij, G^R_ji,
 // G^<>_ij and their conjugate transposes) go from registers to HBM without
-// an LDS slot.
+// an LDS slot.  A round's product takes 2250 cycles, 1536 of them MFMAs; the rest is what a single
+// wave per SIMD cannot put beside them (the FP64 adds of 3M, 7.8 cycles each,
+// LDS and issue).  The blocks of the next backward step are loaded a
+// step ahead, a few in each round.
+//
+// Measured (MI355X): 32 blocks of 32 x 32, 1024 energies 8.47 -> 5.1 ms, 8 blocks, one energy
+// 488 -> 315 us, against the inversion beside the W products only, loads at the
+// start of each step and accumulators in AGPRs (copied to be read; this file is
+// built with MFMA results in VGPRs).
 //
 // Tile products: v_mfma_f64_16x16x4f64, complex as three real products (3M:
 // ar br, ai bi, (ar + ai)(br + bi)) into three accumulators; the sign of a
@@ -54,8 +70,9 @@ typedef double2 Slot[kB][kLd];
 
 struct SmallShared {
   Slot s[kNS];
-  int piv[kB];          // pivot row of each elimination step
-  int step_of[kB];      // step at which each row was the pivot
+  double2 w[8][kB + 1];  // inversion: pivot rows of a sub-panel
+  int piv[kB];           // inversion: pivot row of each elimination step
+  int q_done;            // blocks whose Q^< (odd: and Q^>) is in LDS, times two
   double red[2][4];
   int job;
 };
@@ -78,10 +95,19 @@ __device__ inline Acc acc_zero() {
   return a;
 }
 
-// acc += (NEG ? -1 : 1) op(A) op(B) over KS k-steps of 4 for this wave's tile
-// (tr, tc); op = plain or conjugate transpose (AH / BH).  With op(A) =
-// (ar, sa ai) and op(B) = (br, sb bi): P1 += ar br, P2 += sa sb ai bi,
-// P3 += (ar + sa ai)(br + sb bi), each negated for NEG.  All fragments are read
+// acc += (NEG ? -1 : 1) op(A) op(B) over one k-step of 4; op = plain or conjugate
+// transpose (AH / BH).  With op(A) = (ar, sa ai) and op(B) = (br, sb bi): P1 +=
+// ar br, P2 += sa sb ai bi, P3 += (ar + sa ai)(br + sb bi), each negated for NEG.
+template <bool AH, bool BH, bool NEG>
+__device__ inline void mma_step(Acc& c, double2 a, double2 b) {
+  const double sa = AH ? a.x - a.y : a.x + a.y;
+  const double sb = BH ? b.x - b.y : b.x + b.y;
+  c.p1 = mf<NEG>(a.x, b.x, c.p1);
+  c.p2 = mf<NEG != (AH != BH)>(a.y, b.y, c.p2);
+  c.p3 = mf<NEG>(sa, sb, c.p3);
+}
+
+// The same over KS k-steps for this wave's tile (tr, tc).  All fragments are read
 // before the first MFMA, so the MFMA chain does not wait on LDS.
 template <int KS, bool AH, bool BH, bool NEG>
 __device__ inline void mma(Acc& c, const Slot& A, const Slot& B, int tr, int tc, int lane) {
@@ -95,13 +121,7 @@ __device__ inline void mma(Acc& c, const Slot& A, const Slot& B, int tr, int tc,
     b[s] = BH ? B[col][kk] : B[kk][col];
   }
 #pragma unroll
-  for (int s = 0; s < KS; ++s) {
-    const double sa = AH ? a[s].x - a[s].y : a[s].x + a[s].y;
-    const double sb = BH ? b[s].x - b[s].y : b[s].x + b[s].y;
-    c.p1 = mf<NEG>(a[s].x, b[s].x, c.p1);
-    c.p2 = mf<NEG != (AH != BH)>(a[s].y, b[s].y, c.p2);
-    c.p3 = mf<NEG>(sa, sb, c.p3);
-  }
+  for (int s = 0; s < KS; ++s) mma_step<AH, BH, NEG>(c, a[s], b[s]);
 }
 
 // Register r of a lane holds tile element (4 r + lane / 16, lane % 16).
@@ -112,30 +132,28 @@ __device__ inline void tile_vals(const Acc& c, double2 (&v)[4]) {
 
 __device__ inline int tile_row(int tr, int r, int lane) { return tr * 16 + 4 * r + (lane >> 4); }
 __device__ inline int tile_col(int tc, int lane) { return tc * 16 + (lane & 15); }
-// Tile of product p of a round computed by `wave`.
+// Tile of product p of a round computed by `wave`: with every block above 16 (kFull)
+// the same one for all products, which then share operand fragments; else
+// rotated, so that products with a single live tile spread over the waves.
+template <bool kFull>
 __device__ inline void tile_of(int p, int wave, int& tr, int& tc) {
-  const int t = (wave - p) & 3;
+  const int t = kFull ? wave : (wave - p) & 3;
   tr = t >> 1;
   tc = t & 1;
 }
 
-// Global-memory accesses through address-space-1 pointers: global (not
-// flat) instructions, which count on the vector-memory counter only, so an
-// LDS wait does not also wait for prefetches still in flight.
-typedef __attribute__((address_space(1))) double gdouble;
-__device__ inline double2 gget(const double2* p, int64_t i) {
-  const gdouble* q = (const gdouble*)p + 2 * i;
-  return cmk(q[0], q[1]);
+// Global memory is accessed by buffer loads and stores: an element outside its
+// block has an offset beyond the buffer, which reads as zero and is not
+// written, so that no access needs a branch.  (They count on the vector-memory counter
+// only: an LDS wait does not also wait for prefetches still in flight.)
+__device__ inline unsigned goff(int ld, int rows, int cols, int r, int c) {
+  return r < rows && c < cols ? 16u * (unsigned)(r * ld + c) : kOob;
 }
-__device__ inline void gput(double2* p, int64_t i, double2 v) {
-  gdouble* q = (gdouble*)p + 2 * i;
-  q[0] = v.x;
-  q[1] = v.y;
-}
+__device__ inline void gput(double2* p, int64_t i, double2 v) { buf_store(buf_of(p), 16u * (unsigned)i, v); }
 
-// Element of a global block (row-major, ld), zero outside rows x cols.
+// Element of a global block (row-major, ld), zero outside rows x cols and without a block.
 __device__ inline double2 gld(const double2* F, int ld, int rows, int cols, int r, int c) {
-  return (F && r < rows && c < cols) ? gget(F, (int64_t)r * ld + c) : cmk(0.0, 0.0);
+  return buf_load(buf_of(F), goff(ld, F ? rows : 0, cols, r, c), 0);
 }
 
 // One product's epilogue ingredients: up to three addends
@@ -176,6 +194,7 @@ struct Dst {
   double2* gt = nullptr;
   int ldt = 0;
   double ts = 1.0;
+  double2* keep = nullptr;  // this thread's four elements (registers)
   __device__ Dst glob(double2* p, int ld_, int rows_, int cols_, double s = 1.0) const {
     Dst d = *this;
     d.g = p;
@@ -193,6 +212,10 @@ struct Dst {
     return d;
   }
 };
+__device__ inline Dst kept(Dst d, double2* keep) {
+  d.keep = keep;
+  return d;
+}
 __device__ inline Dst to_slot(int s) {
   Dst d;
   d.slot = s;
@@ -202,9 +225,8 @@ __device__ inline Dst to_glob(double2* p, int ld, int rows, int cols, double s =
   return Dst{}.glob(p, ld, rows, cols, s);
 }
 
-// A product of a round: D (m x n valid) = terms + addends.  `partial`: the
-// value after the first `partial_after` addends also goes there (padded
-// 32 x 32 layout, global).  `on` = false skips the product (uniform).
+// A product of a round: D (m x n valid) = terms + addends.  `on` = false skips
+// the product (uniform).
 template <typename T>
 struct Prod {
   bool on;
@@ -212,64 +234,62 @@ struct Prod {
   T terms;  // void(Acc&, int tr, int tc, int lane)
   Dst d;
   Add a0, a1, a2;
-  double2* partial;
-  int partial_after;
 };
 template <typename T>
 __device__ inline Prod<T> prod(int m, int n, T terms, Dst d, Add a0 = add_none(), Add a1 = add_none(),
-                               Add a2 = add_none(), double2* partial = nullptr, int partial_after = 0,
-                               bool on = true) {
-  return Prod<T>{on, m, n, terms, d, a0, a1, a2, partial, partial_after};
+                               Add a2 = add_none(), bool on = true) {
+  return Prod<T>{on, m, n, terms, d, a0, a1, a2};
 }
 
-template <int I, typename T>
+template <bool kFull, int I, typename T>
 __device__ inline void compute(const Prod<T>& p, double2 (&v)[4], int wave, int lane) {
   int tr, tc;
-  tile_of(I, wave, tr, tc);
-  Acc acc = acc_zero();
-  if (p.on && tr * 16 < p.m && tc * 16 < p.n) p.terms(acc, tr, tc, lane);
-  tile_vals(acc, v);
+  tile_of<kFull>(I, wave, tr, tc);
   if (!p.on) return;
+  if (kFull || (tr * 16 < p.m && tc * 16 < p.n)) {
+    Acc acc = acc_zero();
+    p.terms(acc, tr, tc, lane);
+    tile_vals(acc, v);
+  } else {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = cmk(0.0, 0.0);
+  }
   const Add adds[3] = {p.a0, p.a1, p.a2};
   const int col = tile_col(tc, lane);
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
-    if (p.partial && a == p.partial_after) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) gput(p.partial, tile_row(tr, r, lane) * kB + col, v[r]);
-    }
 #pragma unroll
     for (int r = 0; r < 4; ++r) v[r] = cadd(v[r], add_val(adds[a], r, tile_row(tr, r, lane), col));
   }
 }
 
-template <int I, typename T>
+template <bool kFull, int I, typename T>
 __device__ inline void emit(SmallShared& sh, const Prod<T>& p, const double2 (&v)[4], int wave,
                             int lane) {
   if (!p.on) return;
   int tr, tc;
-  tile_of(I, wave, tr, tc);
+  tile_of<kFull>(I, wave, tr, tc);
   const int col = tile_col(tc, lane);
   const Dst& d = p.d;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int row = tile_row(tr, r, lane);
+    if (d.keep) d.keep[r] = v[r];
     if (d.slot >= 0) sh.s[d.slot][row][col] = v[r];
-    if (d.g && row < d.rows && col < d.cols)
-      gput(d.g, (int64_t)row * d.ld + col, cmk(d.gs * v[r].x, d.gs * v[r].y));
-    if (d.gt && row < d.rows && col < d.cols)
-      gput(d.gt, (int64_t)col * d.ldt + row, cmk(d.ts * v[r].x, -d.ts * v[r].y));
+    if (d.g) buf_store(buf_of(d.g), goff(d.ld, d.rows, d.cols, row, col), cmk(d.gs * v[r].x, d.gs * v[r].y));
+    if (d.gt) buf_store(buf_of(d.gt), goff(d.ldt, d.cols, d.rows, col, row), cmk(d.ts * v[r].x, -d.ts * v[r].y));
   }
 }
 
-template <typename... P, size_t... I>
+template <bool kFull, typename... P, size_t... I>
 __device__ inline void round_impl(SmallShared& sh, bool sync_first, std::index_sequence<I...>,
                                   const P&... ps) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   double2 v[sizeof...(P)][4];
-  (compute<I>(ps, v[I], wave, lane), ...);
+  (compute<kFull, I>(ps, v[I], wave, lane), ...);
   if (sync_first) __syncthreads();
-  (emit<I>(sh, ps, v[I], wave, lane), ...);
+  (emit<kFull, I>(sh, ps, v[I], wave, lane), ...);
   __syncthreads();
 }
 
@@ -277,15 +297,15 @@ __device__ inline void round_impl(SmallShared& sh, bool sync_first, std::index_s
 // barrier).  `sync_first`: wait for every wave between computing and writing,
 // needed when an output slot is an operand or slot addend of any product of
 // the round (other than its own elements as an addend).
-template <typename... P>
+template <bool kFull, typename... P>
 __device__ inline void run_round(SmallShared& sh, bool sync_first, const P&... ps) {
-  round_impl(sh, sync_first, std::index_sequence_for<P...>{}, ps...);
+  round_impl<kFull>(sh, sync_first, std::index_sequence_for<P...>{}, ps...);
 }
 
-// Zero-filled loads of global blocks (rows x cols, ld) into slots, with
-// c2 * src2 (same shape; optional) added and `pad` on the diagonal beyond the
-// valid square (the identity pad of a block about to be inverted).  Thread t
-// moves elements t + 256 q (q < 4) of the padded 32 x 32 block.
+// A global block (rows x cols, ld) on its way into a slot, zero-filled, with c2 *
+// src2 (same shape; optional) added and `pad` on the diagonal beyond the valid
+// square (the identity pad of a block about to be inverted).  Thread t moves
+// elements t + 256 q (q < 4) of the padded 32 x 32 block.
 struct Blk {
   int s;
   const double2* src;
@@ -297,27 +317,32 @@ __device__ inline Blk blk(int s, const double2* src, int ld, int rows, int cols,
                           const double2* src2 = nullptr, double c2 = 0.0, double pad = 0.0) {
   return Blk{s, src, ld, rows, cols, src2, c2, pad};
 }
+// Only loads (unless there is a src2): nothing here waits for them.
 __device__ inline void fetch_blk(const Blk& b, double2 (&v)[4]) {
   const int tid = threadIdx.x;
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     const int idx = tid + q * kThreads;
-    const int r = idx >> 5, c = idx & 31;
-    double2 x = gld(b.src, b.ld, b.rows, b.cols, r, c);
-    if (b.src2 && r < b.rows && c < b.cols) {
-      const double2 w = gget(b.src2, (int64_t)r * b.ld + c);
-      x = cmk(x.x + b.c2 * w.x, x.y + b.c2 * w.y);
+    v[q] = gld(b.src, b.ld, b.rows, b.cols, idx >> 5, idx & 31);
+  }
+  if (b.src2) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int idx = tid + q * kThreads;
+      const double2 w = gld(b.src2, b.ld, b.rows, b.cols, idx >> 5, idx & 31);
+      v[q] = cmk(v[q].x + b.c2 * w.x, v[q].y + b.c2 * w.y);
     }
-    if (r == c && r >= b.rows) x = cmk(b.pad, 0.0);
-    v[q] = x;
   }
 }
-__device__ inline void commit_blk(SmallShared& sh, int s, const double2 (&v)[4]) {
+__device__ inline void commit_blk(SmallShared& sh, int s, const double2 (&v)[4], int rows = kB, double pad = 0.0) {
   const int tid = threadIdx.x;
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     const int idx = tid + q * kThreads;
-    sh.s[s][idx >> 5][idx & 31] = v[q];
+    const int r = idx >> 5, c = idx & 31;
+    double2 x = v[q];
+    if (pad != 0.0 && r == c && r >= rows) x.x = pad;
+    sh.s[s][r][c] = x;
   }
 }
 // The global loads of all NB blocks are issued before the barrier that
@@ -330,11 +355,32 @@ __device__ inline void load_blks(SmallShared& sh, const Blk (&b)[NB]) {
   for (int i = 0; i < NB; ++i) fetch_blk(b[i], v[i]);
   __syncthreads();  // the slots' previous content may still be read
 #pragma unroll
-  for (int i = 0; i < NB; ++i) commit_blk(sh, b[i].s, v[i]);
+  for (int i = 0; i < NB; ++i) commit_blk(sh, b[i].s, v[i], b[i].rows, b[i].pad);
 }
-__device__ inline void load_blk(SmallShared& sh, int s, const double2* src, int ld, int rows, int cols) {
-  const Blk b[1] = {blk(s, src, ld, rows, cols)};
-  load_blks<1>(sh, b);
+
+// The same by one wave alone: global loads now, the slot written by wave_commit.
+__device__ inline void wave_fetch(double2 (&v)[16], const double2* src, int ld, int rows, int cols, int lane) {
+#pragma unroll
+  for (int q = 0; q < 16; ++q) v[q] = gld(src, ld, rows, cols, 2 * q + (lane >> 5), lane & 31);
+}
+__device__ inline void wave_commit(SmallShared& sh, int s, const double2 (&v)[16], int lane, int rows = kB,
+                                   double pad = 0.0) {
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {
+    const int r = 2 * q + (lane >> 5), c = lane & 31;
+    double2 x = v[q];
+    if (pad != 0.0 && r == c && r >= rows) x.x = pad;
+    sh.s[s][r][c] = x;
+  }
+}
+
+// Global write of the valid part of a square slot by one wave.
+__device__ inline void wave_store_blk(double2* dst, int ld, int b, const Slot& s, int lane) {
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {
+    const int r = 2 * q + (lane >> 5), c = lane & 31;
+    buf_store(buf_of(dst), goff(ld, b, b, r, c), s[r][c]);
+  }
 }
 
 // Global write of a slot's valid part after a barrier.  mode 0: dst = s;
@@ -346,151 +392,294 @@ __device__ inline void store_blk(double2* dst, int ld, int rows, int cols, const
   for (int q = 0; q < kB * kB / kThreads; ++q) {
     const int idx = tid + q * kThreads;
     const int r = idx >> 5, c = idx & 31;
-    if (r < rows && c < cols) {
-      double2 v = s[r][c];
-      if (mode == 2) {
-        const double2 l = s[c][r];
-        v = cmk(0.5 * (v.x - l.x), 0.5 * (v.y + l.y));
-      }
-      gput(dst, (int64_t)r * ld + c, v);
+    double2 v = s[r][c];
+    if (mode == 2) {
+      const double2 l = s[c][r];
+      v = cmk(0.5 * (v.x - l.x), 0.5 * (v.y + l.y));
     }
+    buf_store(buf_of(dst), goff(ld, rows, cols, r, c), v);
   }
 }
 
-// Pivot key of a candidate row: the high word of |re| + |im| (non-negative
-// doubles order like their bit patterns; NaN above infinity), with its low six
-// bits replaced by a marker bit (every candidate key is nonzero) and 31 - row
-// (ties go to the lower row).
-__device__ inline unsigned pivot_key(double2 v, int row) {
-  const unsigned hi = (unsigned)(__double_as_longlong(fabs(v.x) + fabs(v.y)) >> 32);
-  return (hi & ~63u) | 32u | (unsigned)(31 - row);
+// Maximum with the value kCtl (row_shr 1, 2, 4, 8) lanes before, zero where that lies
+// before the row of 16: the four in turn leave the row's maximum in its last lane.
+template <int kCtl>
+__device__ inline unsigned dpp_max(unsigned v) {
+  return max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, kCtl, 0xf, 0xf, true));
 }
 
-// Maximum over each row of 16 lanes, left in the row's last lane (row_shr
-// 1, 2, 4, 8; a lane whose source lies before its row keeps its own value).
-__device__ inline unsigned row_max16(unsigned v) {
-  v = max(v, (unsigned)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x111, 0xf, 0xf, false));
-  v = max(v, (unsigned)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x112, 0xf, 0xf, false));
-  v = max(v, (unsigned)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x114, 0xf, 0xf, false));
-  v = max(v, (unsigned)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x118, 0xf, 0xf, false));
-  return v;
+// v_permlane16_swap: lanes 16-31 and 48-63 of x and lanes 0-15 and 32-47 of y
+// change places; v_permlane32_swap: lanes 32-63 of x and 0-31 of y.
+__device__ inline void swap16(double& x, double& y) {
+  const long long a = __double_as_longlong(x), b = __double_as_longlong(y);
+  const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)a, (unsigned)b, false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(a >> 32), (unsigned)(b >> 32), false, false);
+  x = __longlong_as_double(((long long)hi[0] << 32) | lo[0]);
+  y = __longlong_as_double(((long long)hi[1] << 32) | lo[1]);
+}
+__device__ inline void swap32(double& x, double& y) {
+  const long long a = __double_as_longlong(x), b = __double_as_longlong(y);
+  const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)a, (unsigned)b, false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(a >> 32), (unsigned)(b >> 32), false, false);
+  x = __longlong_as_double(((long long)hi[0] << 32) | lo[0]);
+  y = __longlong_as_double(((long long)hi[1] << 32) | lo[1]);
 }
 
-// Value of lane `addr / 4` of this wave (per-lane address; ds_bpermute).
-__device__ inline double bpermute_d(double x, int addr) {
-  const long long b = __double_as_longlong(x);
-  const int lo = __builtin_amdgcn_ds_bpermute(addr, (int)(b & 0xffffffffll));
-  const int hi = __builtin_amdgcn_ds_bpermute(addr, (int)(b >> 32));
-  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+__device__ inline void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 }
 
-// Pivot of the column whose values lanes of half hc hold in `v` (row l % 32):
-// the unused row of largest key (DPP row maxima of the half's two 16-lane
-// rows); marks it used and returns it with its value (every lane of the
-// wave gets the same).
-__device__ inline int pick_pivot(double2 v, int hc, int n, bool& used, double2& pv) {
-  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
-  unsigned key = (h == hc && r < n && !used) ? pivot_key(v, r) : 0u;
-  key = row_max16(key);
-  const unsigned mx = max((unsigned)__builtin_amdgcn_readlane((int)key, 32 * hc + 15),
-                          (unsigned)__builtin_amdgcn_readlane((int)key, 32 * hc + 31));
-  int p = 31 - (int)(mx & 31u);
-  p = p < n ? p : n - 1;
-  if (r == p) used = true;
-  pv = cmk(readlane_d(v.x, 32 * hc + p), readlane_d(v.y, 32 * hc + p));
-  return p;
-}
-
-// Gauss-Jordan inverse of the n x n valid part of slot ms (identity pad
-// beyond n) with partial pivoting and no row moves, by ONE wave with the
-// matrix in registers (no barrier, so the other waves can work meanwhile):
-// step c eliminates column c with the unused row of largest |re| + |im|
-// (compared on the high word; first row on ties), and the result is permuted
-// back at the end, Out[i][j] = M[pi(i)][pi^-1(j)].  Lane l holds row l % 32,
-// columns 16 (l / 32) .. 16 (l / 32) + 15, rotated by one register position
-// per step (for free: the update writes register k + 1's new value into
-// register k), so that column c is always register 0 of the lanes of its
-// half and the step loop stays rolled with constant register indices.
-// Step c: every lane fetches its half of the pivot row from the pivot lane
-// (ds_bpermute) and its row's column-c value from the other half if needed,
-// and applies
-//   row <- keep row - g prow,  keep = 1, g = m_rc / pivot  (keep = 0,
-//   g = -1/pivot for the pivot row),
-// then sets column c to -g.  The step is software-pipelined: register 1
-// (column c + 1) is updated first and the search and reciprocal of step
-// c + 1 run beside the update of the other fifteen registers (one wave has
-// no other work to hide the search's dependent chain behind: 1630 against
-// 1920 cycles per column measured).  Slot ts is scratch for the permutation
-// back into slot ms.
-__device__ __forceinline__ void invert_wave(SmallShared& sh, int ms, int ts, int n, int* info, int tag,
+// Gauss-Jordan inverse of the n x n valid part of slot ms (identity pad beyond n) in place,
+// with partial pivoting and no row moves, by ONE wave (the others work
+// meanwhile; no barrier).  Column c is eliminated with the unused row of largest |re| + |im|
+// (compared on its high word without six bits, first row on ties): pad rows have
+// zeros in valid columns, so they are picked for pad columns only.
+//
+// Blocked like the larger inversion's panels: 8 columns at a time, the other
+// columns once per sub-panel by MFMA, X += T W with T the sub-panel's result and W the pivot
+// rows of X (which leave X as zeros).  A step is bound by the instructions of one wave (660
+// cycles; 1800 with 16 columns per lane updated in every step), so:
+//  * a lane holds row l % 32 of the sub-panel (both halves the same rows) and the pivot row
+//    comes as scalars: 32 v_readlane at 8 cycles, cheaper than ds_bpermute (11 each)
+//    or a way through LDS;
+//  * every lane forms the reciprocal of its own entry beside the search (DPP maximum)
+//    and the other columns' updates;
+//  * the matrix is held transposed in the MFMA accumulator layout (lane: row 16 rt + l % 16,
+//    register u: column 4 u + l / 16), where one v_permlane16_swap and two v_permlane32_swap
+//    turn four columns into rows, and one v_permlane16_swap turns T into the right operand,
+//    which is also the sub-panel's new content.  Only W goes through LDS.
+// Of 9400 cycles per sub-panel the steps take 5300, the 32 MFMAs 2000, W 1100, the
+// change of layout 600.  NT: 16 x 16 tiles per side (1: n <= 16).
+template <int NT>
+__device__ __forceinline__ void invert_wave(SmallShared& sh, int ms, int n, int* info, int tag,
                                             int64_t energy) {
-  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
-  double2 m[16];
+  constexpr int NU = 4 * NT;  // units of four columns
+  const int lane = threadIdx.x & 63, l16 = lane & 15, kq = lane >> 4, row = lane & 31;
+  const bool low = lane < 32;
+  double xr[NT][NU], xi[NT][NU];
 #pragma unroll
-  for (int k = 0; k < 16; ++k) m[k] = sh.s[ms][r][16 * h + k];
-  bool used = false;
-  double2 pv;
-  int p = pick_pivot(m[0], 0, n, used, pv);
-  double2 inv = pivot_recip(pv);
+  for (int rt = 0; rt < NT; ++rt)
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      const double2 v = sh.s[ms][16 * rt + l16][4 * u + kq];
+      xr[rt][u] = v.x;
+      xi[rt][u] = v.y;
+    }
+  unsigned unused = row < 16 * NT ? ~0u : 0u;
+  int step = row, zero_at = -1;
+  const int panels = (n + 7) >> 3;
 #pragma unroll 1
-  for (int c = 0; c < n; ++c) {
-    const int hc = c >> 4;
-    if (lane == 0) {
-      sh.piv[c] = p;
-      sh.step_of[p] = c;
-      if (pv.x == 0.0 && pv.y == 0.0 && atomicCAS(info, 0, tag) == 0) {
-        info[1] = (int)energy;
-        info[2] = c;
+  for (int s = 0; s < panels; ++s) {
+    // units 0 and 1 into rows
+    double re[8], im[8];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      auto rows = [&](double a, double b, double* t) {
+        swap16(a, b);
+        double a2 = a, b2 = b;
+        swap32(a, a2);
+        swap32(b, b2);
+        t[4 * ks] = a;
+        t[4 * ks + 1] = b;
+        t[4 * ks + 2] = a2;
+        t[4 * ks + 3] = b2;
+      };
+      rows(xr[0][ks], NT > 1 ? xr[NT - 1][ks] : 0.0, re);
+      rows(xi[0][ks], NT > 1 ? xi[NT - 1][ks] : 0.0, im);
+    }
+    int sub = -1, p = 0;
+    unsigned mx = 0;
+    double2 iv = cmk(0.0, 0.0);
+    // The search of the next pivot column (its values x, y in re[0], im[0]) and the
+    // reciprocals of its entries, in stages with beside(k) between them
+    auto search = [&](auto beside) {
+      const double x = re[0], y = im[0];
+      auto stage = [&](auto k) {
+        beside(k);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      const double sum = fabs(x) + fabs(y);
+      double big;
+      asm("v_max_f64 %0, |%1|, |%2|" : "=v"(big) : "v"(x), "v"(y));
+      stage(std::integral_constant<int, 0>{});
+      unsigned key = (((unsigned)(__double_as_longlong(sum) >> 32) & ~63u) | (unsigned)(63 - row)) & unused;
+      const int ex = -__builtin_amdgcn_frexp_exp(big);
+      stage(std::integral_constant<int, 1>{});
+      key = dpp_max<0x111>(key);
+      const double sx = __builtin_amdgcn_ldexp(x, ex), sy = __builtin_amdgcn_ldexp(y, ex);
+      stage(std::integral_constant<int, 2>{});
+      key = dpp_max<0x112>(key);
+      double m = sx * sx;
+      stage(std::integral_constant<int, 3>{});
+      m = fma(sy, sy, m);
+      stage(std::integral_constant<int, 4>{});
+      key = dpp_max<0x114>(key);
+      double r = __builtin_amdgcn_rcp(m);
+      stage(std::integral_constant<int, 5>{});
+      double d = fma(-m, r, 1.0);
+      stage(std::integral_constant<int, 6>{});
+      key = dpp_max<0x118>(key);
+      r = fma(r, d, r);
+      stage(std::integral_constant<int, 7>{});
+      d = fma(-m, r, 1.0);
+      unsigned m0 = (unsigned)__builtin_amdgcn_readlane((int)key, 15);
+      unsigned m1 = NT > 1 ? (unsigned)__builtin_amdgcn_readlane((int)key, 31) : 0u;
+      stage(std::integral_constant<int, 8>{});
+      r = fma(r, d, r);
+      mx = m0 > m1 ? m0 : m1;
+      p = 31 - (int)(mx & 31u);
+      stage(std::integral_constant<int, 9>{});
+      double ix = sx * r, iy = -sy * r;
+      stage(std::integral_constant<int, 10>{});
+      ix = __builtin_amdgcn_ldexp(ix, ex);
+      iy = __builtin_amdgcn_ldexp(iy, ex);
+      stage(std::integral_constant<int, 11>{});
+      iv = cmk(readlane_d(ix, p), readlane_d(iy, p));
+    };
+    search([](auto) {});
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      double2 pv[8];
+#pragma unroll
+      for (int q = 1; q < 8; ++q) pv[q] = cmk(readlane_d(re[q], p), readlane_d(im[q], p));
+      double ax = re[0], ay = im[0];
+      if (mx < 64u) {  // (a pivot of zero or next to it)
+        if (row == p && ax == 0.0 && ay == 0.0 && 8 * s + j < n) zero_at = 8 * s + j;
+      }
+      // new[q - 1] = row[q] - g prow[q], new[last] = -g with g = a_r / a_p; the
+      // pivot row has a_r = -1 and starts from zero
+      if (row == p) {
+        unused = 0u;
+        step = 8 * s + j;
+        sub = j;
+        ax = -1.0;
+        ay = 0.0;
+#pragma unroll
+        for (int q = 1; q < 8; ++q) re[q] = im[q] = 0.0;
+      }
+      const double gx = ax * iv.x - ay * iv.y, gy = ax * iv.y + ay * iv.x;
+      double ur = 0.0, ui = 0.0;
+      auto inner = [&](int q) {
+        ur = fma(gy, pv[q].y, re[q]);
+        ui = fma(-gy, pv[q].x, im[q]);
+      };
+      auto outer = [&](int q) {
+        re[q - 1] = fma(-gx, pv[q].x, ur);
+        im[q - 1] = fma(-gx, pv[q].y, ui);
+      };
+      inner(1);
+      outer(1);
+      if (j < 7) {
+        search([&](auto k) {
+          constexpr int q = 2 + decltype(k)::value / 2;
+          if constexpr (decltype(k)::value % 2 == 0) inner(q);
+          else outer(q);
+        });
+      } else {
+#pragma unroll
+        for (int q = 2; q < 8; ++q) {
+          inner(q);
+          outer(q);
+        }
+      }
+      re[7] = -gx;
+      im[7] = -gy;
+    }
+    // the pivot rows leave the other columns and leave zeros
+    {
+      const auto sw = __builtin_amdgcn_permlane16_swap((unsigned)sub, (unsigned)sub, false, false);
+#pragma unroll
+      for (int rt = 0; rt < NT; ++rt) {
+        const int ps = (int)sw[rt];
+        if (ps >= 0) {
+#pragma unroll
+          for (int u = 2; u < NU; ++u) {
+            sh.w[ps][4 * u + kq] = cmk(xr[rt][u], xi[rt][u]);
+            xr[rt][u] = xi[rt][u] = 0.0;
+          }
+        }
       }
     }
-    const int addr = (32 * h + p) * 4;
-    double2 pr[16];
+    // T as the right operand, which is also the new content of its units
+    double tr[2][2], ti[2][2];  // [ks][rt]
 #pragma unroll
-    for (int k = 0; k < 16; ++k) pr[k] = cmk(bpermute_d(m[k].x, addr), bpermute_d(m[k].y, addr));
-    const double ox = __shfl_xor(m[0].x, 32), oy = __shfl_xor(m[0].y, 32);
-    const bool me = r == p;
-    const double2 a = (h == hc) ? m[0] : cmk(ox, oy);  // this row's column-c value
-    const double2 f = cmul(a, inv);
-    const double keep = me ? 0.0 : 1.0;
-    const double2 g = me ? cmk(-inv.x, -inv.y) : f;
-    double2 nw[16];
-    // register 1 holds column c + 1 in the half that owns it
-    nw[1] = cmk(keep * m[1].x - (g.x * pr[1].x - g.y * pr[1].y), keep * m[1].y - (g.x * pr[1].y + g.y * pr[1].x));
-    int pn = p;
-    double2 invn = inv, pvn = pv;
-    if (c + 1 < n) {
-      pn = pick_pivot(nw[1], (c + 1) >> 4, n, used, pvn);
-      invn = pivot_recip(pvn);
+    for (int ks = 0; ks < 2; ++ks) {
+      tr[ks][0] = low ? re[4 * ks] : re[4 * ks + 2];
+      tr[ks][1] = low ? re[4 * ks + 1] : re[4 * ks + 3];
+      ti[ks][0] = low ? im[4 * ks] : im[4 * ks + 2];
+      ti[ks][1] = low ? im[4 * ks + 1] : im[4 * ks + 3];
+      swap16(tr[ks][0], tr[ks][1]);
+      swap16(ti[ks][0], ti[ks][1]);
     }
+    wave_fence();
+    double2 w[2][NT];  // [ks][ct]
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      if (k == 1) continue;
-      nw[k] = cmk(keep * m[k].x - (g.x * pr[k].x - g.y * pr[k].y), keep * m[k].y - (g.x * pr[k].y + g.y * pr[k].x));
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int ct = 0; ct < NT; ++ct) {
+        w[ks][ct] = sh.w[4 * ks + kq][16 * ct + l16];
+        if (ct == 0 && l16 < 8) w[ks][ct] = cmk(0.0, 0.0);
+      }
+    wave_fence();
+    double4_t dr[NT][NT], di[NT][NT];
+#pragma unroll
+    for (int ct = 0; ct < NT; ++ct)
+#pragma unroll
+      for (int rt = 0; rt < NT; ++rt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          dr[rt][ct][r] = xr[rt][4 * ct + r];
+          di[rt][ct][r] = xi[rt][4 * ct + r];
+        }
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int f = 0; f < 4; ++f)
+#pragma unroll
+        for (int ct = 0; ct < NT; ++ct)
+#pragma unroll
+          for (int rt = 0; rt < NT; ++rt) {
+            if (f == 0) dr[rt][ct] = mf<false>(w[ks][ct].x, tr[ks][rt], dr[rt][ct]);
+            if (f == 1) di[rt][ct] = mf<false>(w[ks][ct].x, ti[ks][rt], di[rt][ct]);
+            if (f == 2) dr[rt][ct] = mf<true>(w[ks][ct].y, ti[ks][rt], dr[rt][ct]);
+            if (f == 3) di[rt][ct] = mf<false>(w[ks][ct].y, tr[ks][rt], di[rt][ct]);
+          }
+    // the next sub-panel's units come first
+#pragma unroll
+    for (int rt = 0; rt < NT; ++rt) {
+#pragma unroll
+      for (int u = 0; u < NU - 2; ++u) {
+        xr[rt][u] = dr[rt][(u + 2) >> 2][(u + 2) & 3];
+        xi[rt][u] = di[rt][(u + 2) >> 2][(u + 2) & 3];
+      }
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        xr[rt][NU - 2 + ks] = tr[ks][rt];
+        xi[rt][NU - 2 + ks] = ti[ks][rt];
+      }
     }
-    if (h == hc) nw[0] = cmk(-g.x, -g.y);
-    // rotate by one position
-#pragma unroll
-    for (int k = 0; k < 15; ++k) m[k] = nw[k + 1];
-    m[15] = nw[0];
-    p = pn;
-    pv = pvn;
-    inv = invn;
   }
-  // register k now holds column 16 h + ((k + n) mod 16); permute back
-  // through slot ts: Out[i][j] = M[pi(i)][pi^-1(j)]
+  if (__any(zero_at >= 0)) {
+    int first = zero_at >= 0 ? zero_at : kB;
 #pragma unroll
-  for (int k = 0; k < 16; ++k) sh.s[ts][r][16 * h + ((k + n) & 15)] = m[k];
-  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-  asm volatile("" ::: "memory");
-  const int sr = r < n ? sh.piv[r] : r;
-#pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    const int cc = 16 * h + k;
-    const int sc = cc < n ? sh.step_of[cc] : cc;
-    m[k] = sh.s[ts][sr][sc];
+    for (int o = 16; o > 0; o >>= 1) first = min(first, __shfl_xor(first, o));
+    if (lane == 0 && atomicCAS(info, 0, tag) == 0) {
+      info[1] = (int)energy;
+      info[2] = first;
+    }
   }
+  // units 0 .. NU - 1 now hold columns 8 panels .. in turn; Out[i][j] = M[pi(i)][pi^-1(j)]: row R goes to row step(R), column C to column pi(C)
+  if (low) sh.piv[step & 31] = row;
+  const auto so = __builtin_amdgcn_permlane16_swap((unsigned)step, (unsigned)step, false, false);
+  wave_fence();
+  int pc[NU];
 #pragma unroll
-  for (int k = 0; k < 16; ++k) sh.s[ms][r][16 * h + k] = m[k];
+  for (int u = 0; u < NU; ++u) pc[u] = sh.piv[(4 * u + 8 * panels + kq) & (16 * NT - 1)] & 31;
+#pragma unroll
+  for (int rt = 0; rt < NT; ++rt)
+#pragma unroll
+    for (int u = 0; u < NU; ++u) sh.s[ms][(int)so[rt] & 31][pc[u]] = cmk(xr[rt][u], xi[rt][u]);
 }
 
 // tr(X1 Y1) - tr(X2 Y2) over the valid b x b parts; every thread gets it.
@@ -525,28 +714,158 @@ __device__ double2 trace2(SmallShared& sh, const Slot& X1, const Slot& Y1, const
   return out;
 }
 
-// W = Y A^H + Q^H - Q [= Sigma~, to `partial`] + addends (this lane's
-// elements of all four tiles, in registers), all four tiles by one wave.
+// Fragments of an operand read from a global block (rows x cols, ld) as the
+// right operand of a product: element (4 s + kq, 16 tc + l16), zero outside.
 template <int KS>
-__device__ inline void w_product(SmallShared& sh, int y, int a, int q, int out, int m,
-                                 const double2 (&add)[4][4], double2* partial, int lane) {
+__device__ inline void fetch_right(double2 (&b)[KS / 4][KS], const double2* F, int ld, int rows, int cols, int lane) {
+  const int l16 = lane & 15, kq = lane >> 4;
+#pragma unroll
+  for (int tc = 0; tc < KS / 4; ++tc)
+#pragma unroll
+    for (int s = 0; s < KS; ++s) b[tc][s] = gld(F, ld, rows, cols, 4 * s + kq, 16 * tc + l16);
+}
+
+// All tiles of op(A) op(B) (m x n valid) by one wave, A (and B, unless its fragments
+// are given) in LDS.  Unless kFull, dead tiles are left out (zero).
+template <int KS, bool kFull, bool AH, bool BH>
+__device__ inline void wave_product(double2 (&v)[KS / 4][KS / 4][4], const Slot& A, const Slot* B,
+                                    const double2 (*given)[KS], int m, int n, int lane) {
+  constexpr int NT = KS / 4, H = 4;  // inner steps whose fragments are held at a time
+  const int l16 = lane & 15, kq = lane >> 4;
+  if constexpr (!kFull && NT > 1) {
+#pragma unroll
+    for (int tr = 0; tr < NT; ++tr)
+#pragma unroll
+      for (int tc = 0; tc < NT; ++tc) {
+        if (16 * tr < m && 16 * tc < n) {
+          Acc c = acc_zero();
+#pragma unroll
+          for (int s = 0; s < KS; ++s) {
+            const int kk = 4 * s + kq, x = 16 * tr + l16, y = 16 * tc + l16;
+            mma_step<AH, BH, false>(c, AH ? A[kk][x] : A[x][kk], B ? (BH ? (*B)[y][kk] : (*B)[kk][y]) : given[tc][s]);
+          }
+          tile_vals(c, v[tr][tc]);
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[tr][tc][r] = cmk(0.0, 0.0);
+        }
+      }
+    return;
+  }
+  Acc acc[NT][NT];
+#pragma unroll
+  for (int tr = 0; tr < NT; ++tr)
+#pragma unroll
+    for (int tc = 0; tc < NT; ++tc) acc[tr][tc] = acc_zero();
+#pragma unroll
+  for (int s0 = 0; s0 < KS; s0 += H) {
+    double2 a[NT][H], b[NT][H];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int u = 0; u < H; ++u) {
+        const int kk = (s0 + u) * 4 + kq, x = 16 * t + l16;
+        a[t][u] = AH ? A[kk][x] : A[x][kk];
+        b[t][u] = B ? (BH ? (*B)[x][kk] : (*B)[kk][x]) : given[t][s0 + u];
+      }
+#pragma unroll
+    for (int u = 0; u < H; ++u)
+#pragma unroll
+      for (int tr = 0; tr < NT; ++tr)
+#pragma unroll
+        for (int tc = 0; tc < NT; ++tc) mma_step<AH, BH, false>(acc[tr][tc], a[tr][u], b[tc][u]);
+  }
+#pragma unroll
+  for (int tr = 0; tr < NT; ++tr)
+#pragma unroll
+    for (int tc = 0; tc < NT; ++tc) tile_vals(acc[tr][tc], v[tr][tc]);
+}
+template <int NT>
+__device__ inline void wave_store(SmallShared& sh, int slot, const double2 (&v)[NT][NT][4], int lane) {
+#pragma unroll
+  for (int tr = 0; tr < NT; ++tr)
+#pragma unroll
+    for (int tc = 0; tc < NT; ++tc)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sh.s[slot][tile_row(tr, r, lane)][tile_col(tc, lane)] = v[tr][tc][r];
+}
+
+// The lesser (or greater) part of forward step j by one wave, in place in slot w
+// (W_i on entry, W_j on exit): V = g_i W_i, g^<_i = V g_i^H (to global memory), Y = A_ji
+// g^<_i, W_j = Y A_ji^H + Q^H - Q [= Sigma~, to `partial`] + Sigma_jj + B_j.  Waits for Q
+// before its last product's epilogue.
+template <int KS, bool kFull>
+__device__ inline void lesser_chain(SmallShared& sh, int g, int w, int a, int q, int q_ready, double2* gi, int bi,
+                                    const double2* sd, const double2* ob, int bj, double2* partial, int lane) {
+  constexpr int NT = KS / 4;
+  double2 v[NT][NT][4];
+  wave_product<KS, kFull, false, false>(v, sh.s[g], &sh.s[w], nullptr, bi, bi, lane);
+  wave_fence();
+  wave_store<NT>(sh, w, v, lane);
+  wave_fence();
+  wave_product<KS, kFull, false, true>(v, sh.s[w], &sh.s[g], nullptr, bi, bi, lane);
+  wave_fence();
+  wave_store<NT>(sh, w, v, lane);
+#pragma unroll
+  for (int tr = 0; tr < NT; ++tr)
+#pragma unroll
+    for (int tc = 0; tc < NT; ++tc)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = tile_row(tr, r, lane), col = tile_col(tc, lane);
+        buf_store(buf_of(gi), goff(bi, bi, bi, row, col), v[tr][tc][r]);
+      }
+  // (used by the last product's epilogue)
+  double2 add[NT][NT][4];
+#pragma unroll
+  for (int tr = 0; tr < NT; ++tr)
+#pragma unroll
+    for (int tc = 0; tc < NT; ++tc)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        add[tr][tc][r] = gld(sd, bj, bj, bj, tile_row(tr, r, lane), tile_col(tc, lane));
+  wave_fence();
+  wave_product<KS, kFull, false, false>(v, sh.s[a], &sh.s[w], nullptr, bj, bi, lane);
+  wave_fence();
+  wave_store<NT>(sh, w, v, lane);
+  if (ob) {
+#pragma unroll
+    for (int tr = 0; tr < NT; ++tr)
+#pragma unroll
+      for (int tc = 0; tc < NT; ++tc)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          add[tr][tc][r] = cadd(add[tr][tc][r], gld(ob, bj, bj, bj, tile_row(tr, r, lane), tile_col(tc, lane)));
+  }
+  wave_fence();
+  wave_product<KS, kFull, false, true>(v, sh.s[w], &sh.s[a], nullptr, bj, bj, lane);
+  while (__hip_atomic_load(&sh.q_done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < q_ready)
+    __builtin_amdgcn_s_sleep(1);
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
   const Add qa = add_slot(sh.s[q], -1.0, 1.0);
 #pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const int tr = t >> 1, tc = t & 1;
-    Acc acc = acc_zero();
-    if (tr * 16 < m && tc * 16 < m) mma<KS, false, true, false>(acc, sh.s[y], sh.s[a], tr, tc, lane);
-    double2 v[4];
-    tile_vals(acc, v);
-    const int col = tile_col(tc, lane);
+  for (int tr = 0; tr < NT; ++tr)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = tile_row(tr, r, lane);
-      v[r] = cadd(v[r], add_val(qa, r, row, col));
-      if (partial) gput(partial, row * kB + col, v[r]);
-      sh.s[out][row][col] = cadd(v[r], add[t][r]);
-    }
-  }
+    for (int tc = 0; tc < NT; ++tc)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = tile_row(tr, r, lane), col = tile_col(tc, lane);
+        const double2 x = cadd(v[tr][tc][r], add_val(qa, r, row, col));
+        if (partial) gput(partial, row * kB + col, x);
+        v[tr][tc][r] = cadd(x, add[tr][tc][r]);
+      }
+  wave_store<NT>(sh, w, v, lane);
+}
+
+// Q = P Sigma_ij (from global memory) into slot q by one wave; then announces it.
+template <int KS, bool kFull>
+__device__ inline void q_product(SmallShared& sh, int p, const double2 (&b)[KS / 4][KS], int q, int done, int n,
+                                 int lane) {
+  double2 v[KS / 4][KS / 4][4];
+  wave_product<KS, kFull, false, false>(v, sh.s[p], nullptr, b, n, n, lane);
+  wave_store<KS / 4>(sh, q, v, lane);
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  if (lane == 0) __hip_atomic_store(&sh.q_done, done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
 // Uniform slot allocator (every thread holds the same mask).
@@ -571,285 +890,307 @@ struct Slots {
     mma<KS, AH2, BH2, NEG2>(ac, sh.s[A2], sh.s[B2], tr, tc, lane);                  \
   }
 
+// the problem table and its index tables are read through the scalar
+// (constant) path
+typedef __attribute__((address_space(4))) const SmallProblem cprob;
+
+// One energy point.
+template <int KS, bool kFull>
+__device__ __forceinline__ void sweep_one(SmallShared& sh, const SmallLaunch& L, const cprob& P, int e,
+                                          double2* wg_scratch) {
+  constexpr int NT = KS / 4;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t eg = P.e_base + e;
+  const int N = P.N;
+  const __attribute__((address_space(4))) int* bs = (const __attribute__((address_space(4))) int*)P.bs;
+  const __attribute__((address_space(4))) int64_t* od = (const __attribute__((address_space(4))) int64_t*)P.od;
+  const __attribute__((address_space(4))) int64_t* ou = (const __attribute__((address_space(4))) int64_t*)P.ou;
+  auto D_ = [&](const double2* base, int i) { return base ? base + (int64_t)e * P.Dsz + od[i] : nullptr; };
+  auto U_ = [&](const double2* base, int i) { return base ? base + (int64_t)e * P.Usz + ou[i] : nullptr; };
+  auto Dw = [&](double2* base, int i) { return base ? base + (int64_t)e * P.Dsz + od[i] : nullptr; };
+  auto Uw = [&](double2* base, int i) { return base ? base + (int64_t)e * P.Usz + ou[i] : nullptr; };
+  auto OB = [&](const double2* const* arr, int i) -> const double2* {
+    if (!arr) return nullptr;
+    typedef const double2* cptr;
+    typedef __attribute__((address_space(4))) const cptr ccptr;
+    const double2* b = ((const ccptr*)arr)[i];
+    return b ? b + (int64_t)e * bs[i] * bs[i] : nullptr;
+  };
+  // left-connected g_i: the G^R diagonal output, or this workgroup's scratch
+  double2* gstore = P.GRd ? nullptr : wg_scratch;
+  double2* sigt = wg_scratch ? wg_scratch + (int64_t)(P.GRd ? 0 : N) * kB * kB : nullptr;
+  auto Gd = [&](int i) -> double2* { return P.GRd ? Dw(P.GRd, i) : gstore + (int64_t)i * kB * kB; };
+  auto Gld = [&](int i) { return P.GRd ? bs[i] : kB; };
+  auto SigT = [&](int k, int i) { return sigt + ((int64_t)k * N + i) * kB * kB; };
+  const bool cur = P.cur != nullptr;
+  Slots S;
+
+  // ---- block 0 (rgf.py:216-239): W_0 = Sigma_00 + B_0 ----
+  int cg = S.take(), wl = S.take(), wg = S.take();
+  {
+    const int b = bs[0];
+    const Blk blks[3] = {blk(cg, D_(P.Ad, 0), b, b, b, OB(P.obr, 0), -1.0, 1.0),
+                         blk(wl, D_(P.SLd, 0), b, b, b, OB(P.obl, 0), 1.0),
+                         blk(wg, D_(P.SGd, 0), b, b, b, OB(P.obg, 0), 1.0)};
+    load_blks<3>(sh, blks);
+  }
+  // A_ji, A_ij and A_jj - B^R_j of step j come by wave 2 while block j - 1 is
+  // inverted: the last two into their slots, A_ji into registers
+  int s = S.take(), pp = S.take();
+  const int a = S.take(), t = S.take(), ql = S.take(), qg = S.take();
+  double2 fa[16];
+  auto fetch_step = [&](int j, int slot_s) {
+    const int bi = bs[j - 1], bj = bs[j];
+    double2 fs[16], ft[16];
+    wave_fetch(fs, D_(P.Ad, j), bj, bj, bj, lane);
+    wave_fetch(ft, U_(P.Au, j - 1), bj, bi, bj, lane);  // (bi x bj)
+    wave_fetch(fa, U_(P.Al, j - 1), bi, bj, bi, lane);  // (bj x bi)
+    if (const double2* ob = OB(P.obr, j)) {
+      double2 fo[16];
+      wave_fetch(fo, ob, bj, bj, bj, lane);
+#pragma unroll
+      for (int q = 0; q < 16; ++q) fs[q] = csub(fs[q], fo[q]);
+    }
+    wave_commit(sh, slot_s, fs, lane, bj, 1.0);
+    wave_commit(sh, t, ft, lane);
+  };
+  __syncthreads();
+  if (wave == 3) invert_wave<NT>(sh, cg, bs[0], L.info, 1, eg);
+  if (wave == 2 && N > 1) fetch_step(1, s);
+  __syncthreads();
+
+  // ---- forward sweep (rgf.py:241-302) ----
+  // Only P = A_ji g_i and S = A_jj - B^R_j - P A_ij stand between two inversions:
+  // wave 3 inverts S, and meanwhile waves 0 and 1 take g^<_i and g^>_i from W_i and go on
+  // to W_j (in place), with Q = P Sigma_ij from wave 2, which then stores g_i and brings
+  // the next step's blocks.
+  for (int j = 1; j < N; ++j) {
+    const int i = j - 1;
+    const int bi = bs[i], bj = bs[j];
+    if (wave == 2) wave_commit(sh, a, fa, lane);
+    __syncthreads();
+    run_round<kFull>(sh, false, prod(bj, bi, QX_T(false, false, false, a, cg), to_slot(pp)));
+    run_round<kFull>(sh, false,
+                     prod(bj, bj, QX_T(false, false, true, pp, t), to_slot(s), add_slot(sh.s[s], 1.0)));
+    if (wave == 3) {
+      invert_wave<NT>(sh, s, bj, L.info, j + 1, eg);
+    } else if (wave == 2) {
+      double2 bl[NT][KS], bg[NT][KS];
+      fetch_right<KS>(bl, U_(P.SLu, i), bj, bi, bj, lane);  // Sigma^<_ij
+      fetch_right<KS>(bg, U_(P.SGu, i), bj, bi, bj, lane);  // Sigma^>_ij
+      q_product<KS, kFull>(sh, pp, bl, ql, 2 * j, bj, lane);
+      q_product<KS, kFull>(sh, pp, bg, qg, 2 * j + 1, bj, lane);
+      wave_store_blk(Gd(i), Gld(i), bi, sh.s[cg], lane);
+      if (j + 1 < N) fetch_step(j + 1, pp);
+    } else {
+      const bool gr = wave == 1;
+      lesser_chain<KS, kFull>(sh, cg, gr ? wg : wl, a, gr ? qg : ql, 2 * j + (gr ? 1 : 0),
+                              Dw(gr ? P.GGd : P.GLd, i), bi, D_(gr ? P.SGd : P.SLd, j),
+                              OB(gr ? P.obg : P.obl, j), bj, cur ? SigT(gr ? 1 : 0, j) : nullptr, lane);
+    }
+    __syncthreads();
+    const int g = cg;
+    cg = s;
+    s = pp;
+    pp = g;
+  }
+  store_blk(Gd(N - 1), Gld(N - 1), bs[N - 1], bs[N - 1], sh.s[cg], 0);
+  for (const int x : {a, t, s, pp, ql, qg}) S.give(x);
+  // the backward sweep's input blocks of step i, fetched one step ahead: g_i,
+  // Sigma^<_ij, Sigma^>_ij, A_ij, A_ji
+  double2 pre[5][4];
+  auto fetch_back = [&](int i, int k) {
+    const int bi = bs[i], bj = bs[i + 1];
+    if (k == 0) fetch_blk(blk(0, Gd(i), Gld(i), bi, bi), pre[0]);
+    if (k == 1) fetch_blk(blk(0, U_(P.SLu, i), bj, bi, bj), pre[1]);
+    if (k == 2) fetch_blk(blk(0, U_(P.SGu, i), bj, bi, bj), pre[2]);
+    if (k == 3) fetch_blk(blk(0, U_(P.Au, i), bj, bi, bj), pre[3]);
+    if (k == 4) fetch_blk(blk(0, U_(P.Al, i), bi, bj, bi), pre[4]);
+  };
+  if (N > 1)
+#pragma unroll
+    for (int k = 0; k < 5; ++k) fetch_back(N - 2, k);
+  // V = g W, g^<> = V g^H of the last block
+  {
+    const int b = bs[N - 1], vl = S.take(), vg = S.take();
+    run_round<kFull>(sh, false, prod(b, b, QX_T(false, false, false, cg, wl), to_slot(vl)),
+                     prod(b, b, QX_T(false, false, false, cg, wg), to_slot(vg)));
+    run_round<kFull>(sh, false, prod(b, b, QX_T(false, true, false, vl, cg), to_slot(wl)),
+                     prod(b, b, QX_T(false, true, false, vg, cg), to_slot(wg)));
+    S.give(vl);
+    S.give(vg);
+  }
+  const int cl = wl, cgg = wg;
+
+  // ---- last block: G_{N-1} = g_{N-1}; stored diagonal G^<> projected ----
+  {
+    const int n1 = N - 1, b = bs[n1];
+    store_blk(Dw(P.GLd, n1), b, b, b, sh.s[cl], 2);
+    store_blk(Dw(P.GGd, n1), b, b, b, sh.s[cgg], 2);
+    if (cur) {
+      const int x = S.take(), y = S.take();
+      if (N > 1) {
+        const Blk xy[2] = {blk(x, SigT(1, n1), kB, b, b), blk(y, SigT(0, n1), kB, b, b)};
+        load_blks<2>(sh, xy);
+        __syncthreads();
+        const double2 jv = trace2(sh, sh.s[x], sh.s[cl], sh.s[cgg], sh.s[y], b);
+        if (tid == 0) gput(P.cur, (int64_t)e * (N + 1) + n1, jv);
+      }
+      const Blk xy[2] = {blk(x, OB(P.obg, n1), b, b, b), blk(y, OB(P.obl, n1), b, b, b)};
+      load_blks<2>(sh, xy);
+      __syncthreads();
+      const double2 jn = trace2(sh, sh.s[x], sh.s[cl], sh.s[cgg], sh.s[y], b);
+      if (tid == 0) gput(P.cur, (int64_t)e * (N + 1) + N, cmk(-jn.x, -jn.y));
+      if (N == 1) {
+        // J_0 with the same (first = last) block
+        if (tid == 0) gput(P.cur, (int64_t)e * (N + 1), jn);
+      }
+      S.give(x);
+      S.give(y);
+    }
+  }
+
+  // ---- backward sweep (rgf.py:315-412) ----
+  int X = cg, Xl = cl, Xg = cgg;  // G_jj, G^<>_jj (unprojected)
+  for (int i = N - 2; i >= 0; --i) {
+    const int j = i + 1;
+    const int bi = bs[i], bj = bs[j];
+    // the left-connected g^<>_i (unprojected) are fetched into registers one round
+    // before slots free up for them
+    const int g = S.take(), sgl = S.take(), sgg = S.take(), aij = S.take(), aji = S.take();
+    const Blk gb[2] = {blk(0, Dw(P.GLd, i), bi, bi, bi), blk(0, Dw(P.GGd, i), bi, bi, bi)};
+    double2 gpre[4], gnew[4];
+    commit_blk(sh, g, pre[0]);
+    commit_blk(sh, sgl, pre[1]);
+    commit_blk(sh, sgg, pre[2]);
+    commit_blk(sh, aij, pre[3]);
+    commit_blk(sh, aji, pre[4]);
+    __syncthreads();
+    // Z^<> = g_i Sigma^<>_ij ; U = g_i A_ij ; R = G_jj A_ji (over their B operands)
+    run_round<kFull>(sh, true, prod(bi, bj, QX_T(false, false, false, g, sgl), to_slot(sgl)),
+              prod(bi, bj, QX_T(false, false, false, g, sgg), to_slot(sgg)),
+              prod(bi, bj, QX_T(false, false, false, g, aij), to_slot(aij)),
+              prod(bj, bi, QX_T(false, false, false, X, aji), to_slot(aji)));
+    const int zl = sgl, zg = sgg, u = aij, rr = aji;
+    fetch_blk(gb[0], gpre);
+    // B^<> = Z^<> G_jj^H ; G^R_ij = -U G_jj ; G^R_ji = -R g_i ; K = U R ;
+    // T2^<> = U G^<>_jj (over Z, G_jj and the carried G^<>_jj)
+    run_round<kFull>(sh, true, prod(bi, bj, QX_T(false, true, false, zl, X), to_slot(zl)),
+              prod(bi, bj, QX_T(false, true, false, zg, X), to_slot(zg)),
+              prod(bi, bi, QX_T(false, false, false, u, rr), to_slot(X)),
+              prod(bi, bj, QX_T(false, false, false, u, Xl), to_slot(Xl)),
+              prod(bi, bj, QX_T(false, false, false, u, Xg), to_slot(Xg)),
+              prod(bi, bj, QX_T(false, false, true, u, X), to_glob(Uw(P.GRu, i), bj, bi, bj), add_none(),
+                   add_none(), add_none(), P.GRu != nullptr),
+              prod(bj, bi, QX_T(false, false, true, rr, g), to_glob(Uw(P.GRl, i), bi, bj, bi), add_none(),
+                   add_none(), add_none(), P.GRl != nullptr));
+    const int bl = zl, bg = zg, kk = X, t2l = Xl, t2g = Xg;
+    // g^<_i into the free slot
+    const int gl = S.take();
+    commit_blk(sh, gl, gpre);
+    fetch_blk(gb[1], gpre);
+    __syncthreads();
+    if (i > 0) {
+      fetch_back(i - 1, 0);
+      fetch_back(i - 1, 1);
+    }
+    // G_ii = g_i + K g_i ; G^<_ij = -g^<_i R^H + B^< - T2^< (and G^<_ji =
+    // -(G^<_ij)^H) ; T1^< = K g^<_i - B^< U^H over g_i
+    run_round<kFull>(sh, true,
+              prod(bi, bi, QX_T(false, false, false, kk, g), kept(to_glob(Gd(i), Gld(i), bi, bi), gnew),
+                   add_slot(sh.s[g], 1.0)),
+              prod(bi, bj, QX_T(false, true, true, gl, rr),
+                   to_glob(Uw(P.GLu, i), bj, bi, bj).globT(Uw(P.GLl, i), bi, -1.0), add_slot(sh.s[bl], 1.0),
+                   add_slot(sh.s[t2l], -1.0)),
+              prod(bi, bi, QX_T2(false, false, false, kk, gl, false, true, true, bl, u), to_slot(g)));
+    const int t1l = g;
+    S.give(bl);
+    // g^>_i into the slot of B^<
+    const int gg = S.take();
+    commit_blk(sh, gg, gpre);
+    __syncthreads();
+    if (i > 0) {
+      fetch_back(i - 1, 2);
+      fetch_back(i - 1, 3);
+    }
+    // G^>_ij, G^>_ji ; T1^> = K g^>_i - B^> U^H over K ;
+    // G^<_ii = g^<_i + T2^< U^H + T1^< - T1^<^H (in place)
+    run_round<kFull>(sh, true,
+              prod(bi, bj, QX_T(false, true, true, gg, rr),
+                   to_glob(Uw(P.GGu, i), bj, bi, bj).globT(Uw(P.GGl, i), bi, -1.0), add_slot(sh.s[bg], 1.0),
+                   add_slot(sh.s[t2g], -1.0)),
+              prod(bi, bi, QX_T2(false, false, false, kk, gg, false, true, true, bg, u), to_slot(kk)),
+              prod(bi, bi, QX_T(false, true, false, t2l, u), to_slot(gl), add_slot(sh.s[gl], 1.0),
+                   add_slot(sh.s[t1l], 1.0, -1.0)));
+    const int t1g = kk;
+    if (i > 0) fetch_back(i - 1, 4);
+    // G^>_ii = g^>_i + T2^> U^H + T1^> - T1^>^H (in place)
+    run_round<kFull>(sh, false,
+              prod(bi, bi, QX_T(false, true, false, t2g, u), to_slot(gg), add_slot(sh.s[gg], 1.0),
+                   add_slot(sh.s[t1g], 1.0, -1.0)));
+    store_blk(Dw(P.GLd, i), bi, bi, bi, sh.s[gl], 2);
+    store_blk(Dw(P.GGd, i), bi, bi, bi, sh.s[gg], 2);
+    S.give(t1g);
+    S.give(t1l);
+    S.give(bg);
+    S.give(u);
+    S.give(rr);
+    S.give(t2l);
+    S.give(t2g);
+    Xl = gl;
+    Xg = gg;
+    X = S.take();
+    {
+      int tr, tc;
+      tile_of<kFull>(0, wave, tr, tc);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sh.s[X][tile_row(tr, r, lane)][tile_col(tc, lane)] = gnew[r];
+    }
+    if (cur) {
+      const int x = S.take(), y = S.take();
+      if (i >= 1) {
+        const Blk xy[2] = {blk(x, SigT(1, i), kB, bi, bi), blk(y, SigT(0, i), kB, bi, bi)};
+        load_blks<2>(sh, xy);
+      } else {
+        const Blk xy[2] = {blk(x, OB(P.obg, 0), bi, bi, bi), blk(y, OB(P.obl, 0), bi, bi, bi)};
+        load_blks<2>(sh, xy);
+      }
+      __syncthreads();
+      const double2 jv = trace2(sh, sh.s[x], sh.s[Xl], sh.s[Xg], sh.s[y], bi);
+      if (tid == 0) gput(P.cur, (int64_t)e * (N + 1) + i, jv);
+      S.give(x);
+      S.give(y);
+    }
+  }
+}
+
 template <int KS>
 __global__ void __launch_bounds__(kThreads, 1) sweep_small_kernel(SmallLaunch L) {
   __shared__ SmallShared sh;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   double2* wg_scratch = L.scratch ? (double2*)(L.scratch + (int64_t)blockIdx.x * L.scratch_per_wg) : nullptr;
   for (;;) {
-    if (tid == 0) sh.job = atomicAdd(L.counter, 1);
+    if (threadIdx.x == 0) {
+      sh.job = atomicAdd(L.counter, 1);
+      sh.q_done = 0;
+    }
     __syncthreads();
-    const int job = sh.job;
+    const int job = __builtin_amdgcn_readfirstlane(sh.job);
     __syncthreads();
     if (job >= L.total_jobs) break;
     int p = 0;
-    // the problem table and its index tables are read through the scalar
-    // (constant) path
-    typedef __attribute__((address_space(4))) const SmallProblem cprob;
     const cprob* probs = (const cprob*)L.probs;
     while (p + 1 < L.nprob && job >= probs[p + 1].job0) ++p;
     const cprob& P = probs[p];
     const int e = job - P.job0;
-    const int64_t eg = P.e_base + e;
-    const int N = P.N;
-    const __attribute__((address_space(4))) int* bs = (const __attribute__((address_space(4))) int*)P.bs;
-    const __attribute__((address_space(4))) int64_t* od = (const __attribute__((address_space(4))) int64_t*)P.od;
-    const __attribute__((address_space(4))) int64_t* ou = (const __attribute__((address_space(4))) int64_t*)P.ou;
-    auto D_ = [&](const double2* base, int i) { return base ? base + (int64_t)e * P.Dsz + od[i] : nullptr; };
-    auto U_ = [&](const double2* base, int i) { return base ? base + (int64_t)e * P.Usz + ou[i] : nullptr; };
-    auto Dw = [&](double2* base, int i) { return base ? base + (int64_t)e * P.Dsz + od[i] : nullptr; };
-    auto Uw = [&](double2* base, int i) { return base ? base + (int64_t)e * P.Usz + ou[i] : nullptr; };
-    auto OB = [&](const double2* const* arr, int i) -> const double2* {
-      if (!arr) return nullptr;
-      typedef const double2* cptr;
-      typedef __attribute__((address_space(4))) const cptr ccptr;
-      const double2* b = ((const ccptr*)arr)[i];
-      return b ? b + (int64_t)e * bs[i] * bs[i] : nullptr;
-    };
-    // left-connected g_i: the G^R diagonal output, or this workgroup's scratch
-    double2* gstore = P.GRd ? nullptr : wg_scratch;
-    double2* sigt = wg_scratch ? wg_scratch + (int64_t)(P.GRd ? 0 : N) * kB * kB : nullptr;
-    auto Gd = [&](int i) -> double2* { return P.GRd ? Dw(P.GRd, i) : gstore + (int64_t)i * kB * kB; };
-    auto Gld = [&](int i) { return P.GRd ? bs[i] : kB; };
-    auto SigT = [&](int k, int i) { return sigt + ((int64_t)k * N + i) * kB * kB; };
-    const bool cur = P.cur != nullptr;
-    Slots S;
-
-    // ---- block 0 (rgf.py:216-239) ----
-    int cg, cl, cgg;
-    {
-      const int b = bs[0];
-      cg = S.take();
-      const int w0 = S.take(), w1 = S.take();
-      {
-        const Blk blks[3] = {blk(cg, D_(P.Ad, 0), b, b, b, OB(P.obr, 0), -1.0, 1.0),
-                             blk(w0, D_(P.SLd, 0), b, b, b, OB(P.obl, 0), 1.0),
-                             blk(w1, D_(P.SGd, 0), b, b, b, OB(P.obg, 0), 1.0)};
-        load_blks<3>(sh, blks);
-      }
-      const int vl = S.take(), vg = S.take();
-      __syncthreads();
-      if (wave == 0) invert_wave(sh, cg, vl, b, L.info, 1, eg);
-      __syncthreads();
-      store_blk(Gd(0), Gld(0), b, b, sh.s[cg], 0);
-      // V = g_0 W_0 ; g^<>_0 = V g_0^H (stored unprojected: the carried value)
-      run_round(sh, false, prod(b, b, QX_T(false, false, false, cg, w0), to_slot(vl)),
-                prod(b, b, QX_T(false, false, false, cg, w1), to_slot(vg)));
-      run_round(sh, false,
-                prod(b, b, QX_T(false, true, false, vl, cg), to_slot(w0).glob(Dw(P.GLd, 0), b, b, b)),
-                prod(b, b, QX_T(false, true, false, vg, cg), to_slot(w1).glob(Dw(P.GGd, 0), b, b, b)));
-      S.give(vl);
-      S.give(vg);
-      cl = w0;
-      cgg = w1;
-    }
-
-    // ---- forward sweep (rgf.py:241-302) ----
-    for (int j = 1; j < N; ++j) {
-      const int i = j - 1;
-      const int bi = bs[i], bj = bs[j];
-      // the step's input blocks in one load: A_ji, A_ij, A_jj - B^R_j,
-      // Sigma^<_ij, Sigma^>_ij; the W addends Sigma^<_jj + B^<_j (wave 0) and
-      // Sigma^>_jj + B^>_j (wave 1) of the lane's elements go to registers
-      const int a = S.take(), t = S.take(), s = S.take(), sgl = S.take(), sgg = S.take();
-      double2 wadd[4][4];
-      {
-        const double2* SD = wave == 0 ? D_(P.SLd, j) : D_(P.SGd, j);
-        const double2* BO = wave == 0 ? OB(P.obl, j) : OB(P.obg, j);
-        if (wave >= 2) SD = BO = nullptr;
-#pragma unroll
-        for (int tt = 0; tt < 4; ++tt) {
-          const int c = tile_col(tt & 1, lane);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int rr = tile_row(tt >> 1, r, lane);
-            wadd[tt][r] = cadd(gld(SD, bj, bj, bj, rr, c), gld(BO, bj, bj, bj, rr, c));
-          }
-        }
-      const Blk b[5] = {blk(a, U_(P.Al, i), bi, bj, bi),              // A_ji (bj x bi)
-                          blk(t, U_(P.Au, i), bj, bi, bj),              // A_ij (bi x bj)
-                          blk(s, D_(P.Ad, j), bj, bj, bj, OB(P.obr, j), -1.0, 1.0),
-                          blk(sgl, U_(P.SLu, i), bj, bi, bj),           // Sigma^<_ij
-                          blk(sgg, U_(P.SGu, i), bj, bi, bj)};          // Sigma^>_ij
-        load_blks<5>(sh, b);
-      }
-      const int pp = S.take();
-      __syncthreads();
-      // P = A_ji g_i ; Y^<> = A_ji g^<>_i over the carried g^<>_i
-      run_round(sh, true, prod(bj, bi, QX_T(false, false, false, a, cg), to_slot(pp)),
-                prod(bj, bi, QX_T(false, false, false, a, cl), to_slot(cl)),
-                prod(bj, bi, QX_T(false, false, false, a, cgg), to_slot(cgg)));
-      S.give(cg);
-      const int yl = cl, yg = cgg;
-      // S = A_jj - B^R_j - P A_ij (in place) ; Q^<> = P Sigma^<>_ij over Sigma_ij
-      run_round(sh, true, prod(bj, bj, QX_T(false, false, true, pp, t), to_slot(s), add_slot(sh.s[s], 1.0)),
-                prod(bj, bj, QX_T(false, false, false, pp, sgl), to_slot(sgl)),
-                prod(bj, bj, QX_T(false, false, false, pp, sgg), to_slot(sgg)));
-      S.give(t);
-      const int ql = sgl, qg = sgg;
-      // g_j = S^-1 by wave 3 while waves 0 and 1 form
-      // W^<> = Y^<> A_ji^H + Q^<>^H - Q^<> [= Sigma~] + Sigma^<>_jj + B^<>_j
-      const int wl = S.take(), wg = S.take();
-      if (wave == 3)
-        invert_wave(sh, s, pp, bj, L.info, j + 1, eg);
-      else if (wave == 0)
-        w_product<KS>(sh, yl, a, ql, wl, bj, wadd, cur ? SigT(0, j) : nullptr, lane);
-      else if (wave == 1)
-        w_product<KS>(sh, yg, a, qg, wg, bj, wadd, cur ? SigT(1, j) : nullptr, lane);
-      __syncthreads();
-      S.give(pp);
-      store_blk(Gd(j), Gld(j), bj, bj, sh.s[s], 0);
-      S.give(a);
-      S.give(yl);
-      S.give(yg);
-      S.give(ql);
-      S.give(qg);
-      // V = g_j W ; g^<>_j = V g_j^H (into the W slots, stored unprojected)
-      const int vl = S.take(), vg = S.take();
-      run_round(sh, false, prod(bj, bj, QX_T(false, false, false, s, wl), to_slot(vl)),
-                prod(bj, bj, QX_T(false, false, false, s, wg), to_slot(vg)));
-      run_round(sh, false,
-                prod(bj, bj, QX_T(false, true, false, vl, s), to_slot(wl).glob(Dw(P.GLd, j), bj, bj, bj)),
-                prod(bj, bj, QX_T(false, true, false, vg, s), to_slot(wg).glob(Dw(P.GGd, j), bj, bj, bj)));
-      S.give(vl);
-      S.give(vg);
-      cg = s;
-      cl = wl;
-      cgg = wg;
-    }
-
-    // ---- last block: G_{N-1} = g_{N-1}; stored diagonal G^<> projected ----
-    {
-      const int n1 = N - 1, b = bs[n1];
-      store_blk(Dw(P.GLd, n1), b, b, b, sh.s[cl], 2);
-      store_blk(Dw(P.GGd, n1), b, b, b, sh.s[cgg], 2);
-      if (cur) {
-        const int x = S.take(), y = S.take();
-        if (N > 1) {
-          const Blk xy[2] = {blk(x, SigT(1, n1), kB, b, b), blk(y, SigT(0, n1), kB, b, b)};
-          load_blks<2>(sh, xy);
-          __syncthreads();
-          const double2 jv = trace2(sh, sh.s[x], sh.s[cl], sh.s[cgg], sh.s[y], b);
-          if (tid == 0) gput(P.cur, (int64_t)e * (N + 1) + n1, jv);
-        }
-        const Blk xy[2] = {blk(x, OB(P.obg, n1), b, b, b), blk(y, OB(P.obl, n1), b, b, b)};
-        load_blks<2>(sh, xy);
-        __syncthreads();
-        const double2 jn = trace2(sh, sh.s[x], sh.s[cl], sh.s[cgg], sh.s[y], b);
-        if (tid == 0) gput(P.cur, (int64_t)e * (N + 1) + N, cmk(-jn.x, -jn.y));
-        if (N == 1) {
-          // J_0 with the same (first = last) block
-          if (tid == 0) gput(P.cur, (int64_t)e * (N + 1), jn);
-        }
-        S.give(x);
-        S.give(y);
-      }
-      S.give(cg);
-    }
-
-    // ---- backward sweep (rgf.py:315-412) ----
-    int Xl = cl, Xg = cgg;
-    for (int i = N - 2; i >= 0; --i) {
-      const int j = i + 1;
-      const int bi = bs[i], bj = bs[j];
-      // the step's input blocks in one load: G_jj (retarded, full), g_i
-      // (left-connected), Sigma^<_ij, Sigma^>_ij, A_ij, A_ji; the left-connected
-      // g^<>_i (unprojected) are fetched into registers one round before
-      // slots free up for them
-      const int X = S.take(), g = S.take(), sgl = S.take(), sgg = S.take(), aij = S.take(),
-                aji = S.take();
-      const Blk gb[2] = {blk(0, Dw(P.GLd, i), bi, bi, bi), blk(0, Dw(P.GGd, i), bi, bi, bi)};
-      double2 gpre[4];
-      {
-        const Blk b[6] = {blk(X, Gd(j), Gld(j), bj, bj), blk(g, Gd(i), Gld(i), bi, bi),
-                          blk(sgl, U_(P.SLu, i), bj, bi, bj), blk(sgg, U_(P.SGu, i), bj, bi, bj),
-                          blk(aij, U_(P.Au, i), bj, bi, bj), blk(aji, U_(P.Al, i), bi, bj, bi)};
-        load_blks<6>(sh, b);
-      }
-      __syncthreads();
-      // Z^<> = g_i Sigma^<>_ij ; U = g_i A_ij ; R = G_jj A_ji (over their B operands)
-      run_round(sh, true, prod(bi, bj, QX_T(false, false, false, g, sgl), to_slot(sgl)),
-                prod(bi, bj, QX_T(false, false, false, g, sgg), to_slot(sgg)),
-                prod(bi, bj, QX_T(false, false, false, g, aij), to_slot(aij)),
-                prod(bj, bi, QX_T(false, false, false, X, aji), to_slot(aji)));
-      const int zl = sgl, zg = sgg, u = aij, rr = aji;
-      fetch_blk(gb[0], gpre);
-      // B^<> = Z^<> G_jj^H ; G^R_ij = -U G_jj ; G^R_ji = -R g_i ; K = U R ;
-      // T2^<> = U G^<>_jj (over Z, G_jj and the carried G^<>_jj)
-      run_round(sh, true, prod(bi, bj, QX_T(false, true, false, zl, X), to_slot(zl)),
-                prod(bi, bj, QX_T(false, true, false, zg, X), to_slot(zg)),
-                prod(bi, bj, QX_T(false, false, true, u, X), to_glob(Uw(P.GRu, i), bj, bi, bj), add_none(),
-                     add_none(), add_none(), nullptr, 0, P.GRu != nullptr),
-                prod(bj, bi, QX_T(false, false, true, rr, g), to_glob(Uw(P.GRl, i), bi, bj, bi), add_none(),
-                     add_none(), add_none(), nullptr, 0, P.GRl != nullptr),
-                prod(bi, bi, QX_T(false, false, false, u, rr), to_slot(X)),
-                prod(bi, bj, QX_T(false, false, false, u, Xl), to_slot(Xl)),
-                prod(bi, bj, QX_T(false, false, false, u, Xg), to_slot(Xg)));
-      const int bl = zl, bg = zg, kk = X, t2l = Xl, t2g = Xg;
-      // g^<_i into the free slot
-      const int gl = S.take();
-      commit_blk(sh, gl, gpre);
-      fetch_blk(gb[1], gpre);
-      __syncthreads();
-      // G_ii = g_i + K g_i ; G^<_ij = -g^<_i R^H + B^< - T2^< (and G^<_ji =
-      // -(G^<_ij)^H) ; T1^< = K g^<_i - B^< U^H over g_i
-      run_round(sh, true,
-                prod(bi, bi, QX_T(false, false, false, kk, g), to_glob(Gd(i), Gld(i), bi, bi),
-                     add_slot(sh.s[g], 1.0)),
-                prod(bi, bj, QX_T(false, true, true, gl, rr),
-                     to_glob(Uw(P.GLu, i), bj, bi, bj).globT(Uw(P.GLl, i), bi, -1.0), add_slot(sh.s[bl], 1.0),
-                     add_slot(sh.s[t2l], -1.0)),
-                prod(bi, bi, QX_T2(false, false, false, kk, gl, false, true, true, bl, u), to_slot(g)));
-      const int t1l = g;
-      S.give(bl);
-      // g^>_i into the slot of B^<
-      const int gg = S.take();
-      commit_blk(sh, gg, gpre);
-      __syncthreads();
-      // G^>_ij, G^>_ji ; T1^> = K g^>_i - B^> U^H over K ;
-      // G^<_ii = g^<_i + T2^< U^H + T1^< - T1^<^H (in place)
-      run_round(sh, true,
-                prod(bi, bj, QX_T(false, true, true, gg, rr),
-                     to_glob(Uw(P.GGu, i), bj, bi, bj).globT(Uw(P.GGl, i), bi, -1.0), add_slot(sh.s[bg], 1.0),
-                     add_slot(sh.s[t2g], -1.0)),
-                prod(bi, bi, QX_T2(false, false, false, kk, gg, false, true, true, bg, u), to_slot(kk)),
-                prod(bi, bi, QX_T(false, true, false, t2l, u), to_slot(gl), add_slot(sh.s[gl], 1.0),
-                     add_slot(sh.s[t1l], 1.0, -1.0)));
-      const int t1g = kk;
-      // G^>_ii = g^>_i + T2^> U^H + T1^> - T1^>^H (in place)
-      run_round(sh, false,
-                prod(bi, bi, QX_T(false, true, false, t2g, u), to_slot(gg), add_slot(sh.s[gg], 1.0),
-                     add_slot(sh.s[t1g], 1.0, -1.0)));
-      store_blk(Dw(P.GLd, i), bi, bi, bi, sh.s[gl], 2);
-      store_blk(Dw(P.GGd, i), bi, bi, bi, sh.s[gg], 2);
-      S.give(t1g);
-      S.give(t1l);
-      S.give(bg);
-      S.give(u);
-      S.give(rr);
-      S.give(t2l);
-      S.give(t2g);
-      Xl = gl;
-      Xg = gg;
-      if (cur) {
-        const int x = S.take(), y = S.take();
-        if (i >= 1) {
-          const Blk xy[2] = {blk(x, SigT(1, i), kB, bi, bi), blk(y, SigT(0, i), kB, bi, bi)};
-          load_blks<2>(sh, xy);
-        } else {
-          const Blk xy[2] = {blk(x, OB(P.obg, 0), bi, bi, bi), blk(y, OB(P.obl, 0), bi, bi, bi)};
-          load_blks<2>(sh, xy);
-        }
-        __syncthreads();
-        const double2 jv = trace2(sh, sh.s[x], sh.s[Xl], sh.s[Xg], sh.s[y], bi);
-        if (tid == 0) gput(P.cur, (int64_t)e * (N + 1) + i, jv);
-        S.give(x);
-        S.give(y);
-      }
-    }
+    if (KS == 8 && P.full)
+      sweep_one<KS, KS == 8>(sh, L, P, e, wg_scratch);
+    else
+      sweep_one<KS, false>(sh, L, P, e, wg_scratch);
     __syncthreads();
   }
 }
+
 
 #undef QX_T
 #undef QX_T2
