@@ -135,25 +135,6 @@ __global__ void shift_kernel(const double2* __restrict__ x, const double2* __res
   }
 }
 
-// eps <- eps + x and s <- eps (the inversion copy), per element of a chunk
-__global__ void eps_merge_kernel(double2* __restrict__ eps, const double2* __restrict__ x,
-                                 double2* __restrict__ s, int64_t count) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const double2 v = cadd(eps[i], x[i]);
-    eps[i] = v;
-    s[i] = v;
-  }
-}
-
-hipError_t launch_eps_merge(double2* eps, const double2* x, double2* s, int64_t count,
-                            hipStream_t st) {
-  if (count == 0) return hipSuccess;
-  const int gx = (int)std::min<int64_t>(4096, (count + 255) / 256);
-  hipLaunchKernelGGL(eps_merge_kernel, dim3(gx), dim3(256), 0, st, eps, x, s, count);
-  return hipGetLastError();
-}
-
 hipError_t launch_shift(const double2* x, const double2* s, double eta, int b, int nE,
                         double2* out, hipStream_t st) {
   if (nE == 0) return hipSuccess;
@@ -261,21 +242,23 @@ int rgf_sancho_rubio_z(rgf_ctx* ctx, int64_t b, int64_t n_energies, const void* 
 
   hipStream_t st = ctx->stream;
   const size_t all = mat * nE;
-  rc = ctx->hip(hipMemcpyAsync(Eps, a_ii, all, hipMemcpyDeviceToDevice, st), "copy a_ii");
-  if (!rc) rc = ctx->hip(hipMemcpyAsync(EpsS, a_ii, all, hipMemcpyDeviceToDevice, st), "copy a_ii");
-  if (!rc) rc = ctx->hip(hipMemcpyAsync(S, a_ii, all, hipMemcpyDeviceToDevice, st), "copy a_ii");
-  if (!rc) rc = ctx->hip(hipMemcpyAsync(Al[0], a_ji, all, hipMemcpyDeviceToDevice, st), "copy a_ji");
-  if (!rc) rc = ctx->hip(hipMemcpyAsync(Be[0], a_ij, all, hipMemcpyDeviceToDevice, st), "copy a_ij");
+  rc = ctx->hip(hipMemcpyAsync(S, a_ii, all, hipMemcpyDeviceToDevice, st), "copy a_ii");
   if (!rc) rc = ctx->reset_info();
+  double* host_delta = nullptr;
+  if (!rc) rc = ctx->host_words(nE * sizeof(double), (void**)&host_delta);
   if (rc) return rc;
 
-  std::vector<double> host_delta(nE);
   auto M = [&](double2* p, int64_t e0) { return Mat{p + e0 * bb, bb, n}; };
   int cur = 0;
   int done = 0;
   double dmax = NAN;
   for (int it = 0; it < max_iterations; ++it) {
     const int nxt = cur ^ 1;
+    // the first iteration reads the inputs where they are
+    double2* eps = it ? Eps : (double2*)a_ii;
+    double2* eps_s = it ? EpsS : (double2*)a_ii;
+    double2* al = it ? Al[cur] : (double2*)a_ji;
+    double2* be = it ? Be[cur] : (double2*)a_ij;
     for (int64_t e0 = 0; e0 < nE; e0 += chunk) {
       const int E = (int)std::min<int64_t>(chunk, nE - e0);
       // inverse = inv(epsilon)  (S holds a copy of epsilon; inverted in place)
@@ -283,56 +266,62 @@ int rgf_sancho_rubio_z(rgf_ctx* ctx, int64_t b, int64_t n_energies, const void* 
       if (rc) return rc;
       // alpha g, beta g
       std::vector<ZProblem> p1 = {
-          PB(n, n).term(M(Al[cur], e0), kOpN, Mat{G, bb, n}, kOpN, n).out(Mat{P1, bb, n}).done(),
-          PB(n, n).term(M(Be[cur], e0), kOpN, Mat{G, bb, n}, kOpN, n).out(Mat{P2, bb, n}).done()};
+          PB(n, n).term(M(al, e0), kOpN, Mat{G, bb, n}, kOpN, n).out(Mat{P1, bb, n}).done(),
+          PB(n, n).term(M(be, e0), kOpN, Mat{G, bb, n}, kOpN, n).out(Mat{P2, bb, n}).done()};
       rc = ctx->gemm(p1, E, n);
       if (rc) return rc;
       // epsilon_s -= alpha g beta, with -alpha g beta also written to G (free
-      // now: the inverse was last read above); epsilon -= beta g alpha;
-      // alpha <- alpha g alpha, beta <- beta g beta
+      // now: the inverse was last read above); alpha <- alpha g alpha, beta <- beta g beta
       std::vector<ZProblem> p2 = {
-          PB(n, n).term(Mat{P1, bb, n}, kOpN, M(Be[cur], e0), kOpN, n, MONE)
-              .partial_here().add(M(EpsS, e0), ONE).out(M(EpsS, e0))
+          PB(n, n).term(Mat{P1, bb, n}, kOpN, M(be, e0), kOpN, n, MONE)
+              .partial_here().add(M(eps_s, e0), ONE).out(M(EpsS, e0))
               .out2(kD2Partial, Mat{G, bb, n}).done(),
-          PB(n, n).term(Mat{P2, bb, n}, kOpN, M(Al[cur], e0), kOpN, n, MONE)
-              .add(M(Eps, e0), ONE).out(M(Eps, e0)).done(),
-          PB(n, n).term(Mat{P1, bb, n}, kOpN, M(Al[cur], e0), kOpN, n).out(M(Al[nxt], e0)).done(),
-          PB(n, n).term(Mat{P2, bb, n}, kOpN, M(Be[cur], e0), kOpN, n).out(M(Be[nxt], e0)).done()};
+          PB(n, n).term(Mat{P1, bb, n}, kOpN, M(al, e0), kOpN, n).out(M(Al[nxt], e0)).done(),
+          PB(n, n).term(Mat{P2, bb, n}, kOpN, M(be, e0), kOpN, n).out(M(Be[nxt], e0)).done()};
       rc = ctx->gemm(p2, E, n);
       if (rc) return rc;
-      // epsilon -= alpha g beta; S <- epsilon for the next inverse
-      rc = ctx->hip(launch_eps_merge(Eps + e0 * bb, G, S + e0 * bb, (int64_t)E * bb, st), "eps merge");
+      // delta = max_e ||(|alpha| + |beta|)||_F / 2, read on the host (the stopping
+      // rule): on its way while epsilon is updated, so that the next
+      // inversion is queued before the GPU runs out of work (11 iterations of 64
+      // blocks of 208: 50 us each)
+      if (e0 + E == nE) {
+        for (int64_t f0 = 0; f0 < nE; f0 += kMaxLaunchEnergies) {
+          const int F = (int)std::min<int64_t>(kMaxLaunchEnergies, nE - f0);
+          rc = ctx->hip(launch_pair_norms(Al[nxt] + f0 * bb, Be[nxt] + f0 * bb, bb, bb, F, 0,
+                                          part + f0 * kParts * 2, dE + f0, nullptr, st),
+                        "sancho-rubio delta");
+          if (rc) return rc;
+        }
+        rc = ctx->hip(hipMemcpyAsync(host_delta, dE, nE * sizeof(double), hipMemcpyDeviceToHost, st),
+                      "read delta");
+        if (!rc) rc = ctx->hip(hipEventRecord(ctx->ev_read, st), "delta record");
+        if (rc) return rc;
+      }
+      // epsilon <- epsilon - beta g alpha - alpha g beta, and the copy for the next inverse
+      rc = ctx->gemm({PB(n, n).term(Mat{P2, bb, n}, kOpN, M(al, e0), kOpN, n, MONE)
+                          .add(M(eps, e0), ONE).add(Mat{G, bb, n}, ONE).partial_here()
+                          .out(M(Eps, e0)).out2(kD2Partial, M(S, e0)).done()},
+                     E, n);
       if (rc) return rc;
     }
     cur = nxt;
-    // delta = max_e ||(|alpha| + |beta|)||_F / 2, read on the host (the stopping rule)
-    for (int64_t e0 = 0; e0 < nE; e0 += kMaxLaunchEnergies) {
-      const int E = (int)std::min<int64_t>(kMaxLaunchEnergies, nE - e0);
-      rc = ctx->hip(launch_pair_norms(Al[cur] + e0 * bb, Be[cur] + e0 * bb, bb, bb, E, 0,
-                                      part + e0 * kParts * 2, dE + e0, nullptr, st),
-                    "sancho-rubio delta");
-      if (rc) return rc;
-    }
-    rc = ctx->hip(hipMemcpyAsync(host_delta.data(), dE, nE * sizeof(double), hipMemcpyDeviceToHost, st),
-                  "read delta");
-    if (!rc) rc = ctx->hip(hipStreamSynchronize(st), "sancho-rubio sync");
+    rc = ctx->hip(hipEventSynchronize(ctx->ev_read), "sancho-rubio sync");
     if (rc) return rc;
     dmax = -INFINITY;
-    for (double d : host_delta) {
-      if (std::isnan(d)) { dmax = NAN; break; }
-      dmax = std::max(dmax, d);
+    for (int64_t e = 0; e < nE; ++e) {
+      if (std::isnan(host_delta[e])) { dmax = NAN; break; }
+      dmax = std::max(dmax, host_delta[e]);
     }
     dmax /= 2;
     done = it + 1;
     if (dmax < convergence_tol) break;
   }
-  // x_ii = inv(epsilon_s)
-  rc = ctx->hip(hipMemcpyAsync(S, EpsS, all, hipMemcpyDeviceToDevice, st), "copy eps_s");
-  if (rc) return rc;
+  // x_ii = inv(epsilon_s)  (in place: S still holds a_ii without an iteration)
+  double2* last = done ? EpsS : S;
   double2* X = static_cast<double2*>(x_ii);
   for (int64_t e0 = 0; e0 < nE; e0 += chunk) {
     const int E = (int)std::min<int64_t>(chunk, nE - e0);
-    rc = ctx->inv(S + e0 * bb, bb, n, E, Mat{X + e0 * bb, bb, n}, aux, 3, e0);
+    rc = ctx->inv(last + e0 * bb, bb, n, E, Mat{X + e0 * bb, bb, n}, aux, 3, e0);
     if (rc) return rc;
   }
   if (iterations) *iterations = done;

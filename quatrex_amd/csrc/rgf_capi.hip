@@ -42,6 +42,11 @@ Ctx::~Ctx() {
   if (side) { (void)hipStreamSynchronize(side); (void)hipStreamDestroy(side); }
   if (ev_fork) (void)hipEventDestroy(ev_fork);
   if (ev_join) (void)hipEventDestroy(ev_join);
+  if (ev_read) {
+    (void)hipEventSynchronize(ev_read);
+    (void)hipEventDestroy(ev_read);
+  }
+  if (host_buf) (void)hipHostFree(host_buf);
   for (auto& t : timed) { event_pool.push_back(t.a); event_pool.push_back(t.b); }
   for (hipEvent_t e : event_pool) (void)hipEventDestroy(e);
   if (ws_owned && ws) (void)hipFree(ws);
@@ -300,6 +305,24 @@ int Ctx::inv(double2* S, int64_t sS, int n, int nE, Mat out, char* aux, int tag,
            "zinv launch");
   if (rc) return rc;
   return prof_end(ev, 8.0 * n * (double)n * n * nE, 1, s);
+}
+
+int Ctx::host_words(size_t bytes, void** out) {
+  if (!ev_read) {
+    const int rc = hip(hipEventCreateWithFlags(&ev_read, hipEventDisableTiming), "event");
+    if (rc) return rc;
+  }
+  if (bytes > host_bytes) {
+    (void)hipEventSynchronize(ev_read);  // (a call that failed may have left a copy on its way)
+    if (host_buf) (void)hipHostFree(host_buf);
+    host_buf = nullptr;
+    host_bytes = 0;
+    const int rc = hip(hipHostMalloc(&host_buf, bytes, hipHostMallocDefault), "pinned words");
+    if (rc) return rc;
+    host_bytes = bytes;
+  }
+  *out = host_buf;
+  return RGF_OK;
 }
 
 int Ctx::fork() {

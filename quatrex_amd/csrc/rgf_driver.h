@@ -83,6 +83,12 @@ struct Ctx {
   bool overlap = true;
   hipStream_t side = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+  // a few words that the host reads while the GPU goes on: pinned, kept, grown on
+  // demand, with the event that says they have come
+  void* host_buf = nullptr;
+  size_t host_bytes = 0;
+  hipEvent_t ev_read = nullptr;
+  int host_words(size_t bytes, void** out);
   int fork();   // side stream waits for the work queued so far on `stream`
   int join();   // `stream` waits for the work queued so far on `side`
 
