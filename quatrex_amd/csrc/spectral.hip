@@ -13,14 +13,14 @@
 //
 // The O(b^3) work runs on the existing kernels: every operator inverse
 // T(z_k)^-1 on the batched Gauss-Jordan kernel, every product on the grouped
-// FP64 MFMA GEMM (the quadrature sums accumulate in its epilogue).  The
-// kernels of this file are the small per-energy parts:
+// FP64 MFMA GEMM.  The kernels of this file are the small per-energy parts:
 //   * beyn_probe_kernel: the probe block Y (uniform [0,1) real and imaginary
 //     parts from a counter-based hash of (seed, energy, row, column));
 //   * operator_kernel: T(z) = sum_n z^n a_n for a chunk of quadrature points;
+//   * moment_kernel: q_0 = sum w z T^-1, q_1 = sum w z^2 T^-1 over a chunk's points;
 //   * jacobi_svd_kernel: one-sided (Hestenes) Jacobi SVD of P_0 (b x m_0),
-//     one workgroup per energy, columns rotated in pairs by a round-robin
-//     tournament (one pair per wave at a time);
+//     one workgroup per energy, columns in LDS where they fit, rotated in pairs by
+//     a round-robin tournament (one pair per wave at a time);
 //   * hqr_eig_kernel: eigenpairs of the reduced m x m matrix (m <= 64), one
 //     wave per energy: Householder reduction to Hessenberg form, complex
 //     single-shift QR with Wilkinson shifts and deflation to the Schur form,
@@ -47,6 +47,8 @@ constexpr double2 MONE = {-1.0, 0.0};
 constexpr int kMaxModes = 64;      // m_0 limit of the reduced eigenproblem (one wave)
 constexpr int kMaxCoef = 7;        // polynomial terms n = -3..3
 constexpr int kPtsPerLaunch = 16;  // quadrature points assembled per operator launch
+constexpr int kSvdWaves = 16;      // waves of an SVD workgroup at most
+constexpr size_t kSvdLds = 88 * 1024;  // its column copy in LDS, beside the 67 KB it always takes
 
 __device__ inline double cabs1(double2 a) { return fabs(a.x) + fabs(a.y); }
 __device__ inline double cabs(double2 a) { return hypot(a.x, a.y); }
@@ -65,10 +67,38 @@ __device__ inline double2 csqrt_(double2 a) {
   return cmk(re, im);
 }
 
+// Sum over the wave, in every lane: within rows of 16 lanes by DPP (neighbours, pairs,
+// mirrored half rows, mirrored rows), then across rows by the lane swaps; a
+// shuffle through LDS takes five times as long per step.
+template <int kCtl>
+__device__ inline double dpp_add(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, kCtl, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), kCtl, 0xf, 0xf, true);
+  return v + __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
 __device__ inline double wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-  return v;
+  v = dpp_add<0xb1>(v);
+  v = dpp_add<0x4e>(v);
+  v = dpp_add<0x141>(v);
+  v = dpp_add<0x140>(v);
+  auto both = [](unsigned l0, unsigned h0, unsigned l1, unsigned h1) {
+    return __longlong_as_double(((long long)h0 << 32) | l0) + __longlong_as_double(((long long)h1 << 32) | l1);
+  };
+  long long b = __double_as_longlong(v);
+  auto lo = __builtin_amdgcn_permlane16_swap((unsigned)b, (unsigned)b, false, false);
+  auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
+  v = both(lo[0], hi[0], lo[1], hi[1]);
+  b = __double_as_longlong(v);
+  lo = __builtin_amdgcn_permlane32_swap((unsigned)b, (unsigned)b, false, false);
+  hi = __builtin_amdgcn_permlane32_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
+  return both(lo[0], hi[0], lo[1], hi[1]);
+}
+// |a| without over- or underflow of the squares.
+__device__ inline double cabs_scaled(double2 a) {
+  const int ex = __builtin_amdgcn_frexp_exp(fmax(fabs(a.x), fabs(a.y)));
+  const double x = __builtin_amdgcn_ldexp(a.x, -ex), y = __builtin_amdgcn_ldexp(a.y, -ex);
+  return __builtin_amdgcn_ldexp(sqrt(x * x + y * y), ex);
 }
 __device__ inline double wave_max(double v) {
 #pragma unroll
@@ -107,15 +137,53 @@ struct OpArgs {
   double2* out;                          // [point][energy][d*d]
 };
 
+// Bound by writing T: a thread reads an element's coefficients once for all points of the
+// launch (16 points x 32 energies of 128 x 128: 30 us, 42 with a workgroup per point).
 __global__ void __launch_bounds__(256) operator_kernel(OpArgs P) {
-  const int q = blockIdx.y;  // point * nE + energy
-  const int pt = q / P.nE, e = q % P.nE;
-  double2* o = P.out + (int64_t)q * P.dd;
+  const int e = blockIdx.y;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < P.dd;
        i += (int64_t)gridDim.x * blockDim.x) {
-    double2 v = cmk(0.0, 0.0);
-    for (int n = 0; n < P.ncoef; ++n) v = cadd(v, cmul(P.zp[pt][n], P.a[n][(int64_t)e * P.sA + i]));
-    o[i] = v;
+    double2 a[kMaxCoef];
+#pragma unroll
+    for (int n = 0; n < kMaxCoef; ++n)
+      if (n < P.ncoef) a[n] = P.a[n][(int64_t)e * P.sA + i];
+    double2* o = P.out + (int64_t)e * P.dd + i;
+    for (int pt = 0; pt < P.npts; ++pt) {
+      double2 v = cmk(0.0, 0.0);
+#pragma unroll
+      for (int n = 0; n < kMaxCoef; ++n)
+        if (n < P.ncoef) v = cadd(v, cmul(P.zp[pt][n], a[n]));
+      o[(int64_t)pt * P.nE * P.dd] = v;
+    }
+  }
+}
+
+// Q_0 (+)= sum_j c0_j T_j^-1, Q_1 (+)= sum_j c1_j T_j^-1 over a launch's quadrature points.
+// Bound by reading the inverses once (16 points x 32 energies of 128 x 128, 134 MB:
+// 27 us).
+struct MomentArgs {
+  const double2* tinv;  // [point][energy][d*d]
+  int64_t sP, dd;       // strides of a point and of an energy
+  double2 c0[kPtsPerLaunch], c1[kPtsPerLaunch];
+  int npts, first;
+  double2 *q0, *q1;
+};
+
+__global__ void __launch_bounds__(256) moment_kernel(MomentArgs P) {
+  const int64_t at = (int64_t)blockIdx.y * P.dd;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < P.dd;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    double2 s0 = P.first ? cmk(0.0, 0.0) : P.q0[at + i];
+    double2 s1 = P.first ? cmk(0.0, 0.0) : P.q1[at + i];
+    const double2* t = P.tinv + at + i;
+#pragma unroll 8
+    for (int j = 0; j < P.npts; ++j) {
+      const double2 v = t[j * P.sP];
+      s0 = cadd(s0, cmul(P.c0[j], v));
+      s1 = cadd(s1, cmul(P.c1[j], v));
+    }
+    P.q0[at + i] = s0;
+    P.q1[at + i] = s1;
   }
 }
 
@@ -123,18 +191,25 @@ __global__ void __launch_bounds__(256) operator_kernel(OpArgs P) {
 // column-major scratch copy (m x d per energy).  Outputs, compacted to the
 // r singular values above s_max * m * eps in decreasing order (zero beyond r):
 // U (d x m, unit columns), V (m x m), s (m), rank[e] = r.
-__global__ void __launch_bounds__(256)
+// Bound by the latency of a pair's rotation (read two columns, four sums over the
+// wave, write them back) times rounds times sweeps: a wave per pair of a round, up to
+// 16, and the scratch copy in LDS where it fits (kLds) instead of global memory (128 x
+// 16, 32 energies: 580 us with 4 waves, global memory and shuffles, 441 without
+// the first two, 354 with the sums by DPP).
+template <bool kLds>
+__global__ void __launch_bounds__(1024)
 jacobi_svd_kernel(const double2* __restrict__ P0, double2* __restrict__ A, int d, int m,
                   double2* __restrict__ U, double2* __restrict__ V, double* __restrict__ s_out,
                   int* __restrict__ rank, int max_sweeps) {
   __shared__ double2 Vl[kMaxModes][kMaxModes + 1];  // column-major: Vl[col][row]
-  __shared__ double off_w[4];
+  __shared__ double off_w[kSvdWaves];
   __shared__ double sv[kMaxModes];
   __shared__ int perm[kMaxModes];
   __shared__ int r_sh;
-  const int e = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  extern __shared__ __align__(16) double2 a_lds[];
+  const int e = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = blockDim.x >> 6;
   const double2* P = P0 + (int64_t)e * d * m;
-  double2* Ae = A + (int64_t)e * d * m;
+  double2* Ae = kLds ? a_lds : A + (int64_t)e * d * m;
   double fro = 0.0;
   for (int64_t i = tid; i < (int64_t)d * m; i += blockDim.x) {
     const int r = (int)(i / m), c = (int)(i % m);
@@ -151,14 +226,16 @@ jacobi_svd_kernel(const double2* __restrict__ P0, double2* __restrict__ A, int d
   __syncthreads();
   // columns below eps ||P_0||_F stay below the rank cut (s_max m eps >=
   // sqrt(m) eps ||P_0||_F): they take part in no rotation
-  const double floor2 = DBL_EPSILON * DBL_EPSILON * (off_w[0] + off_w[1] + off_w[2] + off_w[3]);
+  double fro_all = 0.0;
+  for (int w = 0; w < nw; ++w) fro_all += off_w[w];
+  const double floor2 = DBL_EPSILON * DBL_EPSILON * fro_all;
   __syncthreads();
   const int mp = m + (m & 1);
   const double tol = sqrt((double)d) * DBL_EPSILON;
   for (int sweep = 0; sweep < max_sweeps; ++sweep) {
     double off = 0.0;
     for (int t = 0; t < mp - 1; ++t) {
-      for (int k = wave; k < mp / 2; k += 4) {
+      for (int k = wave; k < mp / 2; k += nw) {
         const int pa = k, pb = mp - 1 - k;
         const int p = pa == 0 ? 0 : ((pa - 1 + t) % (mp - 1)) + 1;
         const int q = ((pb - 1 + t) % (mp - 1)) + 1;
@@ -177,7 +254,7 @@ jacobi_svd_kernel(const double2* __restrict__ P0, double2* __restrict__ A, int d
         be = wave_sum(be);
         gr = wave_sum(gr);
         gi = wave_sum(gi);
-        const double g = hypot(gr, gi);
+        const double g = cabs_scaled(cmk(gr, gi));
         if (al <= floor2 || be <= floor2 || g == 0.0) continue;
         const double rel = g / (sqrt(al) * sqrt(be));
         off = fmax(off, rel);
@@ -205,12 +282,13 @@ jacobi_svd_kernel(const double2* __restrict__ P0, double2* __restrict__ A, int d
     }
     if (lane == 0) off_w[wave] = off;
     __syncthreads();
-    const double offall = fmax(fmax(off_w[0], off_w[1]), fmax(off_w[2], off_w[3]));
+    double offall = 0.0;
+    for (int w = 0; w < nw; ++w) offall = fmax(offall, off_w[w]);
     __syncthreads();
     if (offall <= tol) break;
   }
   // singular values (column norms), one wave per column
-  for (int c = wave; c < m; c += 4) {
+  for (int c = wave; c < m; c += nw) {
     double n2 = 0.0;
     for (int r = lane; r < d; r += 64) {
       const double2 x = Ae[(int64_t)c * d + r];
@@ -629,11 +707,8 @@ int beyn_chunk(Ctx* c, int d, int E, int64_t e_glob, const double2* const* coef,
   const int m = bo->m_0;
   const int64_t dd = (int64_t)d * d, dm = (int64_t)d * m, mm = (int64_t)m * m;
   hipStream_t st = c->stream;
-  int rc = c->hip(launch_fill_zero(w.P0, dm, dm, E, st), "zero P0");
-  if (!rc) rc = c->hip(launch_fill_zero(w.P1, dm, dm, E, st), "zero P1");
-  if (rc) return rc;
   hipLaunchKernelGGL(beyn_probe_kernel, grid2(dm, E), dim3(256), 0, st, w.Y, dm, bo->seed, e_glob);
-  rc = c->hip(hipGetLastError(), "probe");
+  int rc = c->hip(hipGetLastError(), "probe");
   if (rc) return rc;
   // quadrature nodes: outer circle (weight + w), inner circle (weight - w)
   const int nq = bo->num_quad_points;
@@ -675,33 +750,51 @@ int beyn_chunk(Ctx* c, int d, int E, int64_t e_glob, const double2* const* coef,
       A.nE = E;
       A.dd = dd;
       A.out = w.T + (int64_t)l0 * E * dd;
-      hipLaunchKernelGGL(operator_kernel, grid2(dd, nl * E), dim3(256), 0, st, A);
+      hipLaunchKernelGGL(operator_kernel, grid2(dd, E), dim3(256), 0, st, A);
       rc = c->hip(hipGetLastError(), "operator");
       if (rc) return rc;
     }
     rc = c->inv(w.T, dd, d, n * E, Mat{w.Tinv, dd, d}, w.aux_pts, 901, e_glob);
     if (rc) return rc;
-    // P_0 += sum w z T^-1 Y, P_1 += sum w z^2 T^-1 Y, two points per launch
-    for (int i = 0; i < n; i += 2) {
-      PB b0(d, m), b1(d, m);
-      for (int j = i; j < std::min(i + 2, n); ++j) {
-        const double2 z = zs[p0 + j];
-        const double s = sg[p0 + j] * wq;
-        const double2 c0{s * z.x, s * z.y};
-        const double2 c1 = hmul(c0, z);
-        const Mat Ti{w.Tinv + (int64_t)j * E * dd, dd, d};
-        b0.term(Ti, kOpN, Mat{w.Y, dm, m}, kOpN, d, c0);
-        b1.term(Ti, kOpN, Mat{w.Y, dm, m}, kOpN, d, c1);
+    // q_0 += sum w z T^-1, q_1 += sum w z^2 T^-1 (in Xij and S, which are used
+    // after the contour)
+    for (int l0 = 0; l0 < n; l0 += kPtsPerLaunch) {
+      MomentArgs A{};
+      A.npts = std::min(kPtsPerLaunch, n - l0);
+      A.tinv = w.Tinv + (int64_t)l0 * E * dd;
+      A.sP = (int64_t)E * dd;
+      A.dd = dd;
+      A.first = p0 + l0 == 0;
+      A.q0 = w.Xij;
+      A.q1 = w.S;
+      for (int j = 0; j < A.npts; ++j) {
+        const double2 z = zs[p0 + l0 + j];
+        const double s = sg[p0 + l0 + j] * wq;
+        A.c0[j] = double2{s * z.x, s * z.y};
+        A.c1[j] = hmul(A.c0[j], z);
       }
-      std::vector<ZProblem> probs = {b0.add(Mat{w.P0, dm, m}, ONE).out(Mat{w.P0, dm, m}).done(),
-                                     b1.add(Mat{w.P1, dm, m}, ONE).out(Mat{w.P1, dm, m}).done()};
-      rc = c->gemm(probs, E, d);
+      hipLaunchKernelGGL(moment_kernel, grid2(dd, E), dim3(256), 0, st, A);
+      rc = c->hip(hipGetLastError(), "moments");
       if (rc) return rc;
     }
   }
+  // P_0 = q_0 Y, P_1 = q_1 Y (two points per launch, products of their inverses with Y,
+  // took 600 us for the 64 points of 32 energies of 128 x 128: 32 chains of 32 k-tiles on
+  // a workgroup per CU)
+  rc = c->gemm({PB(d, m).term(Mat{w.Xij, dd, d}, kOpN, Mat{w.Y, dm, m}, kOpN, d).out(Mat{w.P0, dm, m}).done(),
+                PB(d, m).term(Mat{w.S, dd, d}, kOpN, Mat{w.Y, dm, m}, kOpN, d).out(Mat{w.P1, dm, m}).done()},
+               E, d);
+  if (rc) return rc;
   // SVD projection and the reduced eigenproblem
-  hipLaunchKernelGGL(jacobi_svd_kernel, dim3(E), dim3(256), 0, st, w.P0, w.Acol, d, m, w.U, w.V, w.sv,
-                     w.rank, 60);
+  const int pairs = (m + 1) / 2;
+  const dim3 svd_threads(64 * std::min(kSvdWaves, std::max(4, pairs)));
+  const size_t svd_lds = (size_t)dm * sizeof(double2);
+  if (svd_lds <= kSvdLds)
+    hipLaunchKernelGGL(jacobi_svd_kernel<true>, dim3(E), svd_threads, svd_lds, st, w.P0, w.Acol, d, m, w.U, w.V,
+                       w.sv, w.rank, 60);
+  else
+    hipLaunchKernelGGL(jacobi_svd_kernel<false>, dim3(E), svd_threads, 0, st, w.P0, w.Acol, d, m, w.U, w.V,
+                       w.sv, w.rank, 60);
   rc = c->hip(hipGetLastError(), "jacobi svd");
   if (rc) return rc;
   rc = c->gemm({PB(d, m).term(Mat{w.P1, dm, m}, kOpN, Mat{w.V, mm, m}, kOpN, m).out(Mat{w.T1, dm, m}).done()},
