@@ -1195,10 +1195,6 @@ __global__ void __launch_bounds__(kThreads, 1) sweep_small_kernel(SmallLaunch L)
 #undef QX_T
 #undef QX_T2
 
-__global__ void reset_counter_kernel(int* c) {
-  if (threadIdx.x == 0) c[0] = 0;
-}
-
 }  // namespace
 
 size_t sweep_small_scratch_per_wg(int n_blocks, bool need_g, bool current) {
@@ -1208,7 +1204,6 @@ size_t sweep_small_scratch_per_wg(int n_blocks, bool need_g, bool current) {
 
 hipError_t launch_sweep_small(const SmallLaunch& L, int grid, hipStream_t stream) {
   if (L.total_jobs == 0) return hipSuccess;
-  hipLaunchKernelGGL(reset_counter_kernel, dim3(1), dim3(64), 0, stream, L.counter);
   if (L.bmax <= 16)
     hipLaunchKernelGGL(sweep_small_kernel<4>, dim3(grid), dim3(kThreads), 0, stream, L);
   else
