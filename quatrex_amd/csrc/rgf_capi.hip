@@ -604,7 +604,10 @@ int sweep_chunk_solve(Ctx* c, const Geo& g, int64_t e0, int E, const SolveIO& io
   // The same products in another order (32 blocks of 256, 64 energies: 120.9 -> 116.1 ms, 16
   // of 128 x 64 11.8 -> 11.0, 20 of 256 x 8, captured, 17.5 -> 16.7).  FP32 products keep
   // the plain order: their Newton steps change g_j after the inversion.
-  const bool ahead = c->overlap && !c->prec32;
+  // Not below 1.5 GFLOP of products per step: the two waits between streams
+  // then cost more than is hidden (us with / without: 6 blocks of 40, 4 energies 695 / 651, of 64 x 16
+  // 925 / 880, of 128 x 2 1663 / 1624; 12 of 77 x 48, 1.75 GFLOP, 3640 / 3890).
+  const bool ahead = c->overlap && !c->prec32 && 80.0 * g.bmax * g.bmax * g.bmax * E >= 1.5e9;
   if (!ahead || N == 1) {
     rc = lesser_greater(0, {});
     if (rc) return rc;
@@ -627,7 +630,7 @@ int sweep_chunk_solve(Ctx* c, const Geo& g, int64_t e0, int E, const SolveIO& io
                             .done();
     const ZProblem pQl = PB(bj, bj).term(P, kOpN, SL.U(i), kOpN, bi).out(Ql).done();
     const ZProblem pQg = PB(bj, bj).term(P, kOpN, SG.U(i), kOpN, bi).out(Qg).done();
-    const bool ovl = c->overlap;
+    const bool ovl = ahead || (c->overlap && c->prec32);
     if (ahead) {
       rc = c->gemm({pP}, E, bj);
       if (!rc) rc = c->gemm({pS}, E, bj);
