@@ -1323,8 +1323,8 @@ def main():
         },
         "roofline": {
             "bound": "mfma",
-            "kernel": f"zgemm_grouped_kernel<{tile_m}, {tile_n}, 0, false, {str(tile_3m).lower()}> "
-                      f"(sweep products)",
+            "kernel": (f"zgemm_grouped_kernel<{tile_m}, {tile_n}, 0, ..> (sweep products)" if tile_3m
+                       else f"zgemm4m_kernel<{tile_m}, {tile_n}, 0, false> (sweep products)"),
             "achieved": round(achieved, 3),
             "peak": FP64_PEAK_TFLOPS,
             "unit": "TFLOP/s",

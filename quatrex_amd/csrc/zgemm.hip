@@ -3,11 +3,11 @@
 // Each launch carries up to kMaxProblems independent problems
 //   D = sum_t alpha_t op(A_t) op(B_t) + sum_a (c1_a F_a + c2_a F_a^H)
 // over nE energies.  Two kernels:
-//  * zgemm3m_kernel (second half of the file), the FP64 products of the
+//  * zgemm_grouped_kernel (second half of the file), the FP64 products of the
 //    sweeps: three real MFMAs per complex product;
-//  * zgemm_grouped_kernel: four real MFMAs (v_mfma_f64_16x16x4f64),
+//  * zgemm4m_kernel: four real MFMAs (v_mfma_f64_16x16x4f64),
 //    re += ar*br - ai*bi, im += ar*bi + ai*br, in FP64 or with FP32 operands.
-// In zgemm_grouped_kernel, tiles of op(A) (TM x TK) and op(B) (TK x TN) are staged through LDS,
+// In zgemm4m_kernel, tiles of op(A) (TM x TK) and op(B) (TK x TN) are staged through LDS,
 // k-major so that every MFMA fragment read is 16 contiguous complex values;
 // conjugation and alpha are applied while staging, so the inner loop is the
 // same for every op combination.  Global loads are issued for the next k-tile
@@ -153,7 +153,7 @@ __device__ inline double4_t mfma_nega(double a, double b, double4_t c) {
 template <int TM, int TN, int kRole, bool kF32>
 __global__ void __launch_bounds__((TileShape<TM, TN, kF32>::kThreads),
                                   (TM * TN > 4096 ? 1 : (TM * TN == 4096 ? 4 : 2)))
-zgemm_grouped_kernel(const ZGroup g) {
+zgemm4m_kernel(const ZGroup g) {
   using S = TileShape<TM, TN, kF32>;
   using LT = typename std::conditional<kF32, float2, double2>::type;
   using AccT = typename std::conditional<kF32, float4_t, double4_t>::type;
@@ -397,7 +397,7 @@ hipError_t launch_cfg(const ZGroup& g0, hipStream_t stream) {
   const int64_t total = (int64_t)per * g.nE;
   if (total == 0) return hipSuccess;
   if (total > 0x7fffffff) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((zgemm_grouped_kernel<TM, TN, kRole, kF32>), dim3((unsigned)total),
+  hipLaunchKernelGGL((zgemm4m_kernel<TM, TN, kRole, kF32>), dim3((unsigned)total),
                      dim3(TileShape<TM, TN, kF32>::kThreads), 0, stream, g);
   return hipGetLastError();
 }
@@ -460,8 +460,8 @@ struct Tile3M {
 // TM x TN output tile, WM x WN waves, at least MINW waves per SIMD.  kRole only
 // separates kernel names in traces: 0 = sweep products, 1 = trailing updates
 // inside the blocked inversion.
-template <int TM, int TN, int WM, int WN, int MINW, int kRole, int kForm>
-__global__ void __launch_bounds__(64 * WM * WN, MINW) zgemm3m_kernel(const ZGroup g) {
+template <int TM, int TN, int kRole, int WM, int WN, int MINW, int kForm>
+__global__ void __launch_bounds__(64 * WM * WN, MINW) zgemm_grouped_kernel(const ZGroup g) {
   if (kRole == 1) __builtin_amdgcn_s_setprio(2);  // the inversion is the longer chain
   using S = Tile3M<TM, TN, WM, WN>;
   constexpr int SI = S::SI, SJ = S::SJ, TK = S::kTK;
@@ -765,13 +765,13 @@ hipError_t launch_3m(const ZGroup& g0, hipStream_t stream, bool plain4m = false)
   const dim3 grid((unsigned)total), block(64 * WM * WN);
   if constexpr (kRole == 1 && TM == 32 && TN == 32) {
     if (plain4m) {
-      hipLaunchKernelGGL((zgemm3m_kernel<TM, TN, WM, WN, MINW, kRole, kPlain4M>), grid, block, 0, stream, g);
+      hipLaunchKernelGGL((zgemm_grouped_kernel<TM, TN, kRole, WM, WN, MINW, kPlain4M>), grid, block, 0, stream, g);
       return hipGetLastError();
     }
   }
-  if (gen) hipLaunchKernelGGL((zgemm3m_kernel<TM, TN, WM, WN, MINW, kRole, kGeneral>), grid, block, 0, stream, g);
-  else if (tail) hipLaunchKernelGGL((zgemm3m_kernel<TM, TN, WM, WN, MINW, kRole, kFastTail>), grid, block, 0, stream, g);
-  else hipLaunchKernelGGL((zgemm3m_kernel<TM, TN, WM, WN, MINW, kRole, kFast>), grid, block, 0, stream, g);
+  if (gen) hipLaunchKernelGGL((zgemm_grouped_kernel<TM, TN, kRole, WM, WN, MINW, kGeneral>), grid, block, 0, stream, g);
+  else if (tail) hipLaunchKernelGGL((zgemm_grouped_kernel<TM, TN, kRole, WM, WN, MINW, kFastTail>), grid, block, 0, stream, g);
+  else hipLaunchKernelGGL((zgemm_grouped_kernel<TM, TN, kRole, WM, WN, MINW, kFast>), grid, block, 0, stream, g);
   return hipGetLastError();
 }
 
