@@ -75,6 +75,23 @@ __device__ inline void buf_store(__amdgpu_buffer_rsrc_t r, unsigned off, double2
   __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4_t, v), r, off, 0, 0);
 }
 
+// Memory that a kernel passes over once: with kNt its lines are not kept in the caches.
+// For launches whose data does not fit the Infinity Cache of 256 MB anyway; a smaller
+// one leaves its results there for the kernels that read them.
+constexpr double kCacheBytes = 256.0 * 1024 * 1024;
+typedef double double2_nt __attribute__((ext_vector_type(2)));
+template <bool kNt>
+__device__ inline double2 load_once(const double2* p) {
+  if constexpr (!kNt) return *p;
+  const double2_nt v = __builtin_nontemporal_load(reinterpret_cast<const double2_nt*>(p));
+  return cmk(v.x, v.y);
+}
+template <bool kNt>
+__device__ inline void store_once(double2* p, double2 v) {
+  if constexpr (!kNt) *p = v;
+  else __builtin_nontemporal_store(double2_nt{v.x, v.y}, reinterpret_cast<double2_nt*>(p));
+}
+
 enum Op : int32_t { kOpN = 0, kOpC = 1 };
 enum D2Mode : int32_t { kD2None = 0, kD2Partial = 1, kD2Copy = 2, kD2ConjT = 3 };
 
