@@ -149,7 +149,9 @@ __device__ inline void tile_of(int p, int wave, int& tr, int& tc) {
 __device__ inline unsigned goff(int ld, int rows, int cols, int r, int c) {
   return r < rows && c < cols ? 16u * (unsigned)(r * ld + c) : kOob;
 }
-__device__ inline void gput(double2* p, int64_t i, double2 v) { buf_store(buf_of(p), 16u * (unsigned)i, v); }
+// Element i of what begins at p: within 2 GiB, so p is an energy's own part of an array.
+__device__ inline void gput(double2* p, int i, double2 v) { buf_store(buf_of(p), 16u * (unsigned)i, v); }
+__device__ void gput(double2* p, int64_t i, double2 v) = delete;
 
 // Element of a global block (row-major, ld), zero outside rows x cols and without a block.
 __device__ inline double2 gld(const double2* F, int ld, int rows, int cols, int r, int c) {
@@ -924,6 +926,7 @@ __device__ __forceinline__ void sweep_one(SmallShared& sh, const SmallLaunch& L,
   auto Gld = [&](int i) { return P.GRd ? bs[i] : kB; };
   auto SigT = [&](int k, int i) { return sigt + ((int64_t)k * N + i) * kB * kB; };
   const bool cur = P.cur != nullptr;
+  double2* current = cur ? P.cur + (int64_t)e * (N + 1) : nullptr;
   Slots S;
 
   // ---- block 0 (rgf.py:216-239): W_0 = Sigma_00 + B_0 ----
@@ -1035,16 +1038,16 @@ __device__ __forceinline__ void sweep_one(SmallShared& sh, const SmallLaunch& L,
         load_blks<2>(sh, xy);
         __syncthreads();
         const double2 jv = trace2(sh, sh.s[x], sh.s[cl], sh.s[cgg], sh.s[y], b);
-        if (tid == 0) gput(P.cur, (int64_t)e * (N + 1) + n1, jv);
+        if (tid == 0) gput(current, n1, jv);
       }
       const Blk xy[2] = {blk(x, OB(P.obg, n1), b, b, b), blk(y, OB(P.obl, n1), b, b, b)};
       load_blks<2>(sh, xy);
       __syncthreads();
       const double2 jn = trace2(sh, sh.s[x], sh.s[cl], sh.s[cgg], sh.s[y], b);
-      if (tid == 0) gput(P.cur, (int64_t)e * (N + 1) + N, cmk(-jn.x, -jn.y));
+      if (tid == 0) gput(current, N, cmk(-jn.x, -jn.y));
       if (N == 1) {
         // J_0 with the same (first = last) block
-        if (tid == 0) gput(P.cur, (int64_t)e * (N + 1), jn);
+        if (tid == 0) gput(current, 0, jn);
       }
       S.give(x);
       S.give(y);
@@ -1158,7 +1161,7 @@ __device__ __forceinline__ void sweep_one(SmallShared& sh, const SmallLaunch& L,
       }
       __syncthreads();
       const double2 jv = trace2(sh, sh.s[x], sh.s[Xl], sh.s[Xg], sh.s[y], bi);
-      if (tid == 0) gput(P.cur, (int64_t)e * (N + 1) + i, jv);
+      if (tid == 0) gput(current, i, jv);
       S.give(x);
       S.give(y);
     }

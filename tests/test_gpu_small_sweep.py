@@ -67,3 +67,38 @@ def test_column_scales_leave_the_inverse_alone(device, b):
     scaled = ((A[0].reshape(2, b, b) * d).reshape(2, b * b), *A[1:])
     got = _run(g, scaled, SL, SG, None, device)[0][0].reshape(2, b, b)
     np.testing.assert_array_equal(got * d[:, None], ref)
+
+
+def test_current_of_more_energies_than_two_gib_hold(device):
+    """One 1 x 1 block and 2^26 + 5 energies: the currents, two per energy, end beyond 2 GiB.
+    Scalars: g = 1 / (a - b^R), g^<> = |g|^2 (s^<> + b^<>), J = b^> g^< - g^> b^< in both
+    slots with opposite signs.  Every value is within some 20 roundings of its terms."""
+    import torch
+
+    from quatrex_amd import solve as S
+
+    E, n = 2**26 + 5, 4096
+    g = Geometry((1,))
+    gen = torch.Generator(device=device)
+    gen.manual_seed(17)
+    u = lambda lo, hi: lo + (hi - lo) * torch.rand(E, dtype=torch.float64, device=device, generator=gen)  # noqa: E731
+    none = torch.empty((E, 0), dtype=torch.complex128, device=device)
+    a = torch.complex(u(-1.0, 1.0), u(0.5, 1.0))
+    br = torch.complex(u(-0.1, 0.1), u(-0.2, -0.1))
+    sl, sg, bl, bg = (1j * u(0.1, 1.0) * k for k in (1, -1, 1, -1))
+    out = [S.packed_empty(g, E, device) for _ in range(2)]
+    cur = torch.full((E, 2), float("nan"), dtype=torch.complex128, device=device)
+    col = lambda x: x.reshape(E, 1)  # noqa: E731
+    ob = [[x.reshape(E, 1, 1)] for x in (br, bl, bg)]
+    print(f"current of {E} energies", flush=True)
+    S.selected_solve(g, (col(a), none, none), (col(sl), none), (col(sg), none), g_lesser=out[0], g_greater=out[1],
+                     obc=ob, current=cur)
+    S.default_context(device).status()
+    assert not bool(torch.isnan(cur.real).any())
+    for part in (slice(0, n), slice(2**26 - n // 2, None)):
+        w = 1.0 / (a[part] - br[part]).abs() ** 2
+        gl, gg = w * (sl[part] + bl[part]), w * (sg[part] + bg[part])
+        j = bg[part] * gl - gg * bl[part]
+        tol = 40 * 2.0**-53 * (bg[part].abs() * gl.abs() + gg.abs() * bl[part].abs())
+        assert bool(((cur[part, 0] - j).abs() <= tol).all())
+        assert bool(((cur[part, 1] + j).abs() <= tol).all())
