@@ -52,7 +52,11 @@ extern "C" {
                                       the one-energy-at-a-time baseline)                      */
 #define RGF_OPT_OVERLAP 6          /* 1 (default): each block inversion runs on a second stream of
                                       default priority, beside the lesser and greater
-                                      products of its own and the previous block            */
+                                      products of its own and the previous block, where
+                                      that pays for the waits between the streams: in
+                                      captured FP64 solves, in mixed precision, and in FP64
+                                      calls with a mean of b_i b_(i+1) n_energies of 1.8e5
+                                      and more.  The results do not depend on it          */
 #define RGF_OPT_PROFILE 4          /* 1: time every sweep GEMM launch and every block inversion
                                       with HIP events on the context stream (0: off)          */
 #define RGF_OPT_PERSISTENT 7       /* 1 (default): FP64 selected solves of geometries whose blocks

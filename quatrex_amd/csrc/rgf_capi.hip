@@ -604,10 +604,18 @@ int sweep_chunk_solve(Ctx* c, const Geo& g, int64_t e0, int E, const SolveIO& io
   // The same products in another order (32 blocks of 256, 64 energies: 120.9 -> 116.1 ms, 16
   // of 128 x 64 11.8 -> 11.0, 20 of 256 x 8, captured, 17.5 -> 16.7).  FP32 products keep
   // the plain order: their Newton steps change g_j after the inversion.
-  // Not below 1.5 GFLOP of products per step: the two waits between streams
-  // then cost more than is hidden (us with / without: 6 blocks of 40, 4 energies 695 / 651, of 64 x 16
-  // 925 / 880, of 128 x 2 1663 / 1624; 12 of 77 x 48, 1.75 GFLOP, 3640 / 3890).
-  const bool ahead = c->overlap && !c->prec32 && 80.0 * g.bmax * g.bmax * g.bmax * E >= 1.5e9;
+  // A call that is not being captured pays two waits between streams in every step, 15 to 20
+  // us.  What they hide grows with the step's products, and a product's time grows only once
+  // it fills the chip: so not below 1.8e5 elements (180 tiles of 32 x 32 for 256
+  // CUs) of a product, in the mean over the steps.  Time plain / ahead, 8 equal blocks: 33 x 70
+  // energies 0.97, x 139 1.03; 48 x 45 0.96, x 79 1.005; 64 x 33 0.99, x 72 1.03; 96 x 14 0.98, x 21
+  // 1.004; 128 x 6 0.98, x 13 1.000; 192 x 2 0.98, x 4 0.997; 256 x 1 0.99, x 4 0.99; 512 x 1 1.01.
+  // Unequal: (40, 40, 200) x 2, 8 energies 0.95, 32 1.02; (33 x 5, 256) x 2, 8 0.94, 32 0.99;
+  // (94, 60, 80, 66, 90, 70) x 2, 16 0.99, 32 1.02.
+  // In a graph the waits are edges and cost nothing: 0.995 to 1.14 over all of these.
+  double elems = 0;
+  for (int j = 1; j < N; ++j) elems += (double)g.bs[j - 1] * g.bs[j] * E / (N - 1);
+  const bool ahead = c->overlap && !c->prec32 && (c->capturing || elems >= 1.8e5);
   if (!ahead || N == 1) {
     rc = lesser_greater(0, {});
     if (rc) return rc;
@@ -1902,6 +1910,7 @@ int rgf_graph_capture_solve(rgf_ctx* ctx, const rgf_geometry* geom, int64_t n_en
   ctx->profile = false;
   ctx->prec32 = mixed;
   ctx->refine = mixed ? refine : 0;
+  ctx->capturing = true;
   // Capture is recorded on a private stream (the caller's stream may be the
   // legacy NULL stream, which cannot be captured); the graph is launched on
   // the context's stream.
@@ -1927,6 +1936,7 @@ int rgf_graph_capture_solve(rgf_ctx* ctx, const rgf_geometry* geom, int64_t n_en
   ctx->profile = saved_prof;
   ctx->prec32 = saved32;
   ctx->refine = saved_ref;
+  ctx->capturing = false;
   if (rc_sweep) rc = rc_sweep;
   if (!rc) rc = ctx->hip(hipGraphInstantiate(&gr->exec, graph, nullptr, nullptr, 0), "instantiate");
   gr->graph = graph;

@@ -81,6 +81,7 @@ struct Ctx {
   // run each block inversion on a second stream, beside the lesser and
   // greater products that do not need it
   bool overlap = true;
+  bool capturing = false;  // a graph is being recorded: its waits cost the host nothing
   hipStream_t side = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   // a few words that the host reads while the GPU goes on: pinned, kept, grown on

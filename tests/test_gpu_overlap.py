@@ -71,3 +71,76 @@ def test_captured_overlap_replays_the_eager_result(device):
                 assert torch.equal(p, q)
         eager[0][0].abs().sum().item()  # eager work between the replays
     graph.close()
+
+
+def _launches(g, mats, ob, E, ctx, on, device):
+    """Product launches of one solve: the order with overlap has one more per step."""
+    A, SL, SG = mats
+    out = [S.packed_empty(g, E, device) for _ in range(3)]
+    ctx.set_option(_lib.RGF_OPT_OVERLAP, on)
+    ctx.profile(True)
+    try:
+        ctx.profile_read()
+        S.selected_solve(g, A, SL, SG, g_lesser=out[1], g_greater=out[2], g_retarded=out[0], obc=ob)
+        ctx.status()
+        return ctx.profile_read()["gemm_launches"], out
+    finally:
+        ctx.profile(False)
+        ctx.set_option(_lib.RGF_OPT_OVERLAP, 1)
+
+
+@pytest.mark.parametrize("bs,E,two_streams", [
+    ((40, 40, 200), 8, False),           # one wide block: most steps are small
+    ((33, 33, 33, 256), 8, False),
+    ((48, 48, 48), 78, False), ((48, 48, 48), 79, True),  # 179712 and 182016 elements
+    ((65, 33, 96, 34), 70, True), ((40, 65), 80, True), ((512, 512), 1, True),
+])
+def test_second_stream_only_for_products_that_fill_the_chip(device, bs, E, two_streams):
+    import torch
+
+    print(f"overlap rule bs={bs} E={E}", flush=True)
+    n = len(bs)
+    assert (E * sum(a * b for a, b in zip(bs, bs[1:])) / (n - 1) >= 1.8e5) == two_streams
+    g, A, SL, SG, obc = edge_case(bs, seed=sum(bs), E=min(E, 4))
+    t = lambda x: torch.as_tensor(np.ascontiguousarray(np.resize(x, (E, *x.shape[1:]))), device=device)  # noqa: E731
+    mats = [tuple(map(t, m)) for m in (A, SL, SG)]
+    ob = [[None if x is None else t(x) for x in row] for row in obc]
+    ctx = S.default_context(device)
+    plain, ref = _launches(g, mats, ob, E, ctx, 0, device)
+    got, out = _launches(g, mats, ob, E, ctx, 1, device)
+    assert got - plain == (n - 1 if two_streams else 0)
+    for o, r in zip(out, ref):
+        for p, q in zip(o, r):
+            assert torch.equal(p, q)
+
+
+def test_captured_two_stream_sweep_with_current(device):
+    """Large enough that the eager solve runs on two streams too."""
+    import torch
+
+    bs, E = (65, 40, 96), 60
+    assert E * (65 * 40 + 40 * 96) / 2 >= 1.8e5
+    g, _, (A, SL, SG), ob = _device_case(bs, E, device)
+    ref = [S.packed_empty(g, E, device) for _ in range(3)]
+    out = [S.packed_empty(g, E, device) for _ in range(3)]
+    cur = [torch.empty((E, len(bs) + 1), dtype=torch.complex128, device=device) for _ in range(2)]
+    ctx = S.default_context(device)
+    ctx.set_option(_lib.RGF_OPT_OVERLAP, 0)
+    try:
+        S.selected_solve(g, A, SL, SG, g_lesser=ref[1], g_greater=ref[2], g_retarded=ref[0], obc=ob, current=cur[0])
+    finally:
+        ctx.set_option(_lib.RGF_OPT_OVERLAP, 1)
+    graph = S.SolveGraph(g, A, SL, SG, g_lesser=out[1], g_greater=out[2], g_retarded=out[0], obc=ob, current=cur[1])
+    flat = lambda o, c: [p for x in o for p in x] + [c]  # noqa: E731
+    for k in range(4):
+        for p in flat(out, cur[1]):
+            p.zero_()
+        torch.cuda.synchronize()
+        graph.launch()
+        if k == 2:  # the same sweep, eager, right behind the replay
+            S.selected_solve(g, A, SL, SG, g_lesser=out[1], g_greater=out[2], g_retarded=out[0], obc=ob, current=cur[1])
+        torch.cuda.synchronize()
+        for p, q in zip(flat(out, cur[1]), flat(ref, cur[0])):
+            assert torch.equal(p, q)
+        ref[0][0].abs().sum().item()  # eager work between the replays
+    graph.close()
