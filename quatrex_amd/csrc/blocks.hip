@@ -32,16 +32,13 @@ fill_zero_kernel(double2* p, int64_t count, int64_t stride) {
     q[i] = cmk(0.0, 0.0);
 }
 
-// Past the caches (kNt) when a launch moves more than a quarter of them: a call's launches
-// are three parts of up to three stacks (32 blocks of 256, 64 energies, full pattern, 12.6
-// GB: densify 2.66 -> 2.45 ms, sparsify 2.65 -> 2.37; 20 blocks of 96, 64 energies, partly
-// filled, a selected solve on the stacks 9.47 -> 9.33 ms).
-inline bool streams(int64_t n, int nE) { return 32.0 * n * nE > kCacheBytes / 4; }
-
 // Energies per thread: a map entry is loaded once and applied to kEPT
 // energies (the map is shared by all energies of the stack).
 constexpr int kEPT = 8;
 
+// kNt: past the caches, except for mirrored entries.  Those are written down the columns, 16
+// bytes of a line at a time, and only the caches put the lines together (24 x 24 to 256 x 256
+// blocks, all entries stored, symmetric, 3 GB: 0.8-1.1 ms cached, 1.3-2.7 past the caches).
 template <bool kNt>
 __global__ void __launch_bounds__(256)
 densify_kernel(const double2* __restrict__ data, int64_t sData, int64_t n,
@@ -54,15 +51,19 @@ densify_kernel(const double2* __restrict__ data, int64_t sData, int64_t n,
     const int64_t s = src[k], d = dst[k];
     const uint8_t f = op[k];
     for (int u = 0; u < ne; ++u) {
-      const double2 v = load_once<kNt>(&data[(int64_t)(e0 + u) * sData + s]);
-      double2 w = v;
+      const double2* from = &data[(int64_t)(e0 + u) * sData + s];
+      double2* to = &out[(int64_t)(e0 + u) * sOut + d];
       if (f & kMirror) {
-        w = sym_op(v, f);
-      } else if (f & kDiagSym) {
+        *to = sym_op(*from, f);
+        continue;
+      }
+      const double2 v = load_once<kNt>(from);
+      double2 w = v;
+      if (f & kDiagSym) {
         const double2 t = sym_op(v, f);
         w = cmk(0.5 * (v.x + t.x), 0.5 * (v.y + t.y));
       }
-      store_once<kNt>(&out[(int64_t)(e0 + u) * sOut + d], w);
+      store_once<kNt>(to, w);
     }
   }
 }
@@ -100,25 +101,25 @@ hipError_t launch_fill_zero(double2* p, int64_t count, int64_t stride, int nE, h
 
 hipError_t launch_densify(const double2* data, int64_t sData, int64_t n, const int64_t* src,
                           const int64_t* dst, const uint8_t* op, double2* out, int64_t sOut,
-                          int nE, hipStream_t s) {
+                          int nE, bool past_caches, hipStream_t s) {
   if (n <= 0 || nE <= 0) return hipSuccess;
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, grid_for(n, (nE + kEPT - 1) / kEPT), dim3(256), 0, s, data, sData, n, src, dst, op,
                        out, sOut, nE);
   };
-  streams(n, nE) ? go(densify_kernel<true>) : go(densify_kernel<false>);
+  past_caches ? go(densify_kernel<true>) : go(densify_kernel<false>);
   return hipGetLastError();
 }
 
 hipError_t launch_sparsify(const double2* in, int64_t sIn, int64_t n, const int64_t* src,
                            const int64_t* dst, const uint8_t* op, double2* data, int64_t sData,
-                           int nE, hipStream_t s) {
+                           int nE, bool past_caches, hipStream_t s) {
   if (n <= 0 || nE <= 0) return hipSuccess;
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, grid_for(n, (nE + kEPT - 1) / kEPT), dim3(256), 0, s, in, sIn, n, src, dst, op, data,
                        sData, nE);
   };
-  streams(n, nE) ? go(sparsify_kernel<true>) : go(sparsify_kernel<false>);
+  past_caches ? go(sparsify_kernel<true>) : go(sparsify_kernel<false>);
   return hipGetLastError();
 }
 

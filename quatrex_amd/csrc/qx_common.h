@@ -269,13 +269,13 @@ hipError_t launch_sweep_small(const SmallLaunch& L, int grid, hipStream_t stream
 
 // Block-sparse <-> packed tridiagonal (blocks.hip).  Entry k of a map moves
 // data[e][src[k]] to out[e][dst[k]] (densify) or back (sparsify, stored
-// entries only); op flags in blocks.hip.
+// entries only); op flags in blocks.hip.  past_caches: the call moves more than they hold.
 hipError_t launch_fill_zero(double2* p, int64_t count, int64_t stride, int nE, hipStream_t s);
 hipError_t launch_densify(const double2* data, int64_t sData, int64_t n, const int64_t* src,
                           const int64_t* dst, const uint8_t* op, double2* out, int64_t sOut,
-                          int nE, hipStream_t s);
+                          int nE, bool past_caches, hipStream_t s);
 hipError_t launch_sparsify(const double2* in, int64_t sIn, int64_t n, const int64_t* src,
                            const int64_t* dst, const uint8_t* op, double2* data, int64_t sData,
-                           int nE, hipStream_t s);
+                           int nE, bool past_caches, hipStream_t s);
 
 }  // namespace qx

@@ -1961,6 +1961,14 @@ int rgf_graph_destroy(rgf_graph* graph) {
   return RGF_OK;
 }
 
+// Entries per energy that a call moves, all parts.
+static int64_t moved_entries(const rgf_block_map* map, const double2* const (&parts)[3]) {
+  int64_t n = 0;
+  for (int p = 0; p < 3; ++p)
+    if (parts[p]) n += std::max<int64_t>(map->part[p].n, 0);
+  return n;
+}
+
 int rgf_densify_z(rgf_ctx* ctx, const rgf_geometry* geom, int64_t n_energies, const void* data,
                   int64_t data_stride, const rgf_block_map* map, rgf_bt* out) {
   if (!ctx) return RGF_EINVAL;
@@ -1980,6 +1988,12 @@ int rgf_densify_z(rgf_ctx* ctx, const rgf_geometry* geom, int64_t n_energies, co
     if (m.n > 0 && (!parts[p] || !m.src || !m.dst || !m.op))
       return ctx->fail(RGF_EINVAL, "densify: map part without output or index arrays");
   }
+  // Past the caches from one and a half times what they hold on (us cached / past, 16 blocks of 64, 256 / 320 / 500
+  // MB: all entries stored 51 / 52, 73 / 65, 108 / 96, half of them 130 / 140, 158 / 166, 269 / 255).  A
+  // symmetric stack, whose map has more entries than are stored, stays cached: its other
+  // entries meet the mirrored ones in the same lines (all stored, 500 MB: 143 / 178).
+  const int64_t moved = moved_entries(map, {parts[0], parts[1], parts[2]});
+  const bool past = 32.0 * moved * n_energies > 1.5 * qx::kCacheBytes && moved <= data_stride;
   for (int p = 0; p < 3; ++p) {
     if (!parts[p]) continue;
     const rgf_block_map_part& m = map->part[p];
@@ -1988,7 +2002,7 @@ int rgf_densify_z(rgf_ctx* ctx, const rgf_geometry* geom, int64_t n_energies, co
       if (rc) return rc;
     }
     rc = ctx->hip(launch_densify(static_cast<const double2*>(data), data_stride, m.n, m.src, m.dst, m.op,
-                                 parts[p], size[p], (int)n_energies, ctx->stream),
+                                 parts[p], size[p], (int)n_energies, past, ctx->stream),
                   "densify");
     if (rc) return rc;
   }
@@ -2011,12 +2025,17 @@ int rgf_sparsify_z(rgf_ctx* ctx, const rgf_geometry* geom, int64_t n_energies,
   const double2* parts[3] = {static_cast<const double2*>(in->diag), static_cast<const double2*>(in->upper),
                              static_cast<const double2*>(in->lower)};
   const int64_t size[3] = {g.Dsz, g.Usz, g.Usz};
+  // Past the caches when the call moves more than they hold; mirrored entries are not moved (us
+  // cached / past, 16 blocks of 64, 200 / 256 / 320 MB: all entries stored 35 / 42, 51 / 52, 76 / 65, half of them 68 / 64,
+  // 94 / 83, 110 / 101; symmetric, 160 / 250 / 500 MB: 32 / 39, 56 / 55, 116 / 103).
+  const int64_t moved = std::min(moved_entries(map, parts), data_stride);
+  const bool past = 32.0 * moved * n_energies > qx::kCacheBytes;
   for (int p = 0; p < 3; ++p) {
     const rgf_block_map_part& m = map->part[p];
     if (m.n <= 0 || !parts[p]) continue;  // parts not given are left untouched in data
     if (!m.src || !m.dst || !m.op) return ctx->fail(RGF_EINVAL, "sparsify: map part without index arrays");
     rc = ctx->hip(launch_sparsify(parts[p], size[p], m.n, m.src, m.dst, m.op,
-                                  static_cast<double2*>(data), data_stride, (int)n_energies, ctx->stream),
+                                  static_cast<double2*>(data), data_stride, (int)n_energies, past, ctx->stream),
                   "sparsify");
     if (rc) return rc;
   }

@@ -91,3 +91,78 @@ def test_block_moves_past_the_caches(device, layout, symmetry, op):
         sparsify_batch(y, slice(lo, min(lo + 16, E)), g, cut, "dul", device, ctx)
     assert torch.equal(x.data, y.data)
     assert bool(x.data.any())
+
+
+def _calls(c, g, device, ctx, parts, bufs=None):
+    """Densify of all energies in one call, and in slices that the caches hold (or sparsify into c)."""
+    E, step = int(c.data.shape[0]), 32
+    one = lambda lo, hi: (  # noqa: E731
+        densify_batch(c, slice(lo, hi), g, parts, device, ctx, data=c.data[lo:hi])[0] if bufs is None else
+        sparsify_batch(c, slice(lo, hi), g, tuple(p[lo:hi] for p in bufs), parts, device, ctx))
+    return (lambda: one(0, E)), (lambda: [one(lo, min(lo + step, E)) for lo in range(0, E, step)])
+
+
+@pytest.mark.parametrize("parts", ["dul", "d", "l"])
+@pytest.mark.parametrize("symmetry,op", SYMMETRY)
+def test_one_large_move_equals_its_slices(device, parts, symmetry, op):
+    """Past the line of 1.5 times the caches, also for single parts; a symmetric stack's lower
+    part is mirrored whole, its diagonal part half."""
+    import torch
+
+    bs, E = [96, 91, 100, 96, 88, 97, 99, 96], {"dul": 257, "d": 720, "l": 720}[parts]
+    g = Geometry(bs)
+    m = _matrix(bs, 47, symmetry, op)
+    c = DSDBCOO.from_sparray(m, bs, (E,), symmetry, op, device=device)
+    entries = 0.28 * {"dul": g.diag_size + 2 * g.offdiag_size, "d": g.diag_size, "l": g.offdiag_size}[parts]
+    assert 32 * E * entries > 1.5 * 256 * 2**20
+    gen = torch.Generator(device=device)
+    gen.manual_seed(8)
+    c.data.copy_(_random(tuple(c.data.shape), device, gen))
+    ctx = S.default_context(device)
+    whole, sliced = _calls(c, g, device, ctx, parts)
+    a, b = whole(), sliced()
+    for k, x in enumerate(a):
+        if x is not None:
+            assert torch.equal(x, torch.cat([s[k] for s in b]))
+    x, y = DSDBCOO.zeros_like(c), DSDBCOO.zeros_like(c)
+    if parts == "dul":
+        _calls(x, g, device, ctx, parts, a)[0]()
+        _calls(y, g, device, ctx, parts, a)[1]()
+        assert torch.equal(x.data, y.data) and bool(x.data.any())
+
+
+@pytest.mark.parametrize("symmetry", [False, True])
+def test_one_large_move_is_no_slower_than_its_slices(device, symmetry):
+    """A call past the caches against the same energies in cached calls, all entries stored; the slices
+    pass through as much memory and have 16 times the launches.  (Mirrored entries written past
+    the caches took 2.1 times as long.)"""
+    import time
+
+    import torch
+
+    bs, E = (64,) * 16, 512
+    g = Geometry(bs)
+    i, j = np.indices((g.n, g.n), dtype=np.int64).reshape(2, -1)
+    keep = (np.abs(i // 64 - j // 64) <= 1) & ((i <= j) | (not symmetry))
+    i, j = i[keep], j[keep]
+    order = np.lexsort((j, i, j // 64, i // 64))
+    data = torch.ones((E, i.size), dtype=torch.complex128, device=device)
+    c = DSDBCOO(data, i[order], j[order], bs, (E,), symmetry)
+    ctx = S.default_context(device)
+
+    def best(f):
+        f()
+        times = []
+        for _ in range(7):
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            f()
+            torch.cuda.synchronize()
+            times.append(time.perf_counter() - t)
+        return min(times)
+
+    whole, sliced = _calls(c, g, device, ctx, "dul")
+    bufs = whole()
+    assert best(whole) <= 1.3 * best(sliced)
+    whole, sliced = _calls(DSDBCOO.zeros_like(c), g, device, ctx, "dul", bufs)
+    assert best(whole) <= 1.3 * best(sliced)
