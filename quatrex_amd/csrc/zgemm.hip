@@ -418,8 +418,8 @@ hipError_t launch_cfg(const ZGroup& g0, hipStream_t stream) {
 //    fragment sums (an fma with a scalar +-1 in the place of the add) and the
 //    sign of P2, and a negative term that of all three; the accumulators keep
 //    the sum up to those signs, are negated where a term's signs differ from
-//    the one before it, and the last signs are applied in the epilogue.  Any
-//    other alpha scales op(A) on its way into LDS (kGeneral).
+//    the one before it, and the last signs are applied in the epilogue.  (No
+//    product has another alpha: the launch refuses it.)
 //  * operands come by buffer loads with one lane offset per element and a scalar
 //    offset per k-tile; rows and columns beyond the edge have an offset beyond
 //    the buffer, which reads as zero, and so have the inner indices beyond K
@@ -444,9 +444,9 @@ hipError_t launch_cfg(const ZGroup& g0, hipStream_t stream) {
 #define QX_SGB(mask, n) __builtin_amdgcn_sched_group_barrier(mask, n, 0)
 constexpr int kSgMfma = 0x8, kSgVmemRead = 0x20, kSgDsRead = 0x100, kSgDsWrite = 0x200;
 
-// kFast: alpha = +-1, every K a multiple of 8; kFastTail: alpha = +-1;
-// kGeneral: any.  kPlain4M: four MFMAs per product (no conjugation, alpha = 1).
-enum Form : int { kFast = 0, kFastTail = 1, kGeneral = 2, kPlain4M = 3 };
+// kFast: every K a multiple of 8; kFastTail: any K; kPlain4M: any K, four MFMAs per
+// product (no conjugation, alpha = 1).
+enum Form : int { kFast = 0, kFastTail = 1, kPlain4M = 2 };
 
 template <int TM, int TN, int WM, int WN>
 struct Tile3M {
@@ -465,7 +465,7 @@ __global__ void __launch_bounds__(64 * WM * WN, MINW) zgemm_grouped_kernel(const
   if (kRole == 1) __builtin_amdgcn_s_setprio(2);  // the inversion is the longer chain
   using S = Tile3M<TM, TN, WM, WN>;
   constexpr int SI = S::SI, SJ = S::SJ, TK = S::kTK;
-  constexpr bool kGen = kForm == kGeneral, kTail = kForm != kFast, k4M = kForm == kPlain4M;
+  constexpr bool kTail = kForm != kFast, k4M = kForm == kPlain4M;
   __shared__ double2 lds_a[2 * TK * S::LA];
   __shared__ double2 lds_b[2 * TK * S::LB];
 
@@ -571,9 +571,8 @@ __global__ void __launch_bounds__(64 * WM * WN, MINW) zgemm_grouped_kernel(const
       kb[i] = bN ? idx / TN : idx % TK;
       offb[i] = gn < n ? 16u * (bN ? kb[i] * ldb + gn : gn * ldb + kb[i]) : kOob;
     }
-    const double2 alpha = T.alpha;
     {
-      const bool t1 = !kGen && alpha.x < 0.0, t2 = t1 != (aN != bN);
+      const bool t1 = T.alpha.x < 0.0, t2 = t1 != (aN != bN);
       if (ti > 0 && t1 != neg1) {
 #pragma unroll
         for (int i = 0; i < SI; ++i)
@@ -617,10 +616,7 @@ __global__ void __launch_bounds__(64 * WM * WN, MINW) zgemm_grouped_kernel(const
     };
     auto store = [&](int buf) {
 #pragma unroll
-      for (int i = 0; i < S::kAPer; ++i) {
-        // (conjugate(a) alpha = conjugate(a conjugate(alpha)): the MFMAs conjugate)
-        wa[i][buf * (TK * S::LA)] = kGen ? cmul(aN ? alpha : cconj(alpha), ra[i]) : ra[i];
-      }
+      for (int i = 0; i < S::kAPer; ++i) wa[i][buf * (TK * S::LA)] = ra[i];
 #pragma unroll
       for (int i = 0; i < S::kBPer; ++i) wb[i][buf * (TK * S::LB)] = rb[i];
     };
@@ -745,7 +741,7 @@ template <int TM, int TN, int WM, int WN, int MINW, int kRole>
 hipError_t launch_3m(const ZGroup& g0, hipStream_t stream, bool plain4m = false) {
   ZGroup g = g0;
   int per = 0;
-  bool gen = false, tail = false;
+  bool unit = true, tail = false;
   for (int p = 0; p < g.nprob; ++p) {
     const int tm = (g.p[p].m + TM - 1) / TM, tn = (g.p[p].n + TN - 1) / TN;
     g.tiles_n[p] = tn;
@@ -754,14 +750,14 @@ hipError_t launch_3m(const ZGroup& g0, hipStream_t stream, bool plain4m = false)
     per += tm * tn;
     for (int t = 0; t < g.p[p].nterms; ++t) {
       const ZTerm& T = g.p[p].t[t];
-      gen |= T.alpha.y != 0.0 || (T.alpha.x != 1.0 && T.alpha.x != -1.0);
+      unit &= T.alpha.y == 0.0 && (T.alpha.x == 1.0 || T.alpha.x == -1.0);
       tail |= T.k % Tile3M<TM, TN, WM, WN>::kTK != 0;
     }
   }
   g.wg_base[g.nprob] = per;
   const int64_t total = (int64_t)per * g.nE;
   if (total == 0) return hipSuccess;
-  if (total > 0x7fffffff) return hipErrorInvalidValue;
+  if (total > 0x7fffffff || !unit) return hipErrorInvalidValue;
   const dim3 grid((unsigned)total), block(64 * WM * WN);
   if constexpr (kRole == 1 && TM == 32 && TN == 32) {
     if (plain4m) {
@@ -769,8 +765,7 @@ hipError_t launch_3m(const ZGroup& g0, hipStream_t stream, bool plain4m = false)
       return hipGetLastError();
     }
   }
-  if (gen) hipLaunchKernelGGL((zgemm_grouped_kernel<TM, TN, kRole, WM, WN, MINW, kGeneral>), grid, block, 0, stream, g);
-  else if (tail) hipLaunchKernelGGL((zgemm_grouped_kernel<TM, TN, kRole, WM, WN, MINW, kFastTail>), grid, block, 0, stream, g);
+  if (tail) hipLaunchKernelGGL((zgemm_grouped_kernel<TM, TN, kRole, WM, WN, MINW, kFastTail>), grid, block, 0, stream, g);
   else hipLaunchKernelGGL((zgemm_grouped_kernel<TM, TN, kRole, WM, WN, MINW, kFast>), grid, block, 0, stream, g);
   return hipGetLastError();
 }
