@@ -13,8 +13,8 @@
 // tridiagonal blocks.
 //
 // Bound by memory: three reads and a write per element.  Past the size of the Infinity
-// Cache they go around the caches (kNt): 32 blocks of 256, 32 energies, 12.6 GB, 2.67 ms
-// (4.7 TB/s) -> 2.36 (5.3); 16 of 64, 64 energies, 0.77 GB, 165 us -> 143; 8 of 64, 64
+// Cache they go around the caches (kNt): 32 blocks of 256, 32 energies, 12.6 GB, 2.55-2.67 ms
+// (4.7-4.9 TB/s) -> 2.30-2.37 (5.3-5.5); 16 of 64, 64 energies, 0.77 GB, 165 us -> 143; 8 of 64, 64
 // energies, 0.37 GB, 91 us -> 74.
 #include <algorithm>
 #include <string>

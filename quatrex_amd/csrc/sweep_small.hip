@@ -42,7 +42,9 @@
 // Measured (MI355X): 32 blocks of 32 x 32, 1024 energies 8.47 -> 5.1 ms, 8 blocks, one energy
 // 488 -> 315 us, against the inversion beside the W products only, loads at the
 // start of each step and accumulators in AGPRs (copied to be read; this file is
-// built with MFMA results in VGPRs).
+// built with MFMA results in VGPRs).  Errors against 64 bits, rms over four seeds, the elimination column
+// by column / in sub-panels: 12 blocks of 16 6.3e-14 / 6.7e-14, 16 of 24 1.09e-13 / 0.86e-13, 8 of 32 8.3e-15 /
+// 8.5e-15, 32 of 32 4.58e-14 / 4.45e-14.
 //
 // Tile products: v_mfma_f64_16x16x4f64, complex as three real products (3M:
 // ar br, ai bi, (ar + ai)(br + bi)) into three accumulators; the sign of a

@@ -3,7 +3,8 @@
 //
 // Step c eliminates column c with pivot row pi(c), the row of largest
 // |re|+|im| among the rows not yet used as pivots (LAPACK izamax's measure,
-// first physical row on ties).  Nothing is swapped: after all steps the matrix
+// first physical row on ties; from 33 to 512 rows compared by its ten highest
+// mantissa bits).  Nothing is swapped: after all steps the matrix
 // holds M with A^{-1}[i][j] = M[pi(i)][pi^{-1}(j)].  A panel of NB columns
 // [k, k+nb) is eliminated by a panel kernel, one workgroup per energy and
 // unblocked GJE on the panel: zinv_panel2_kernel up to 32 rows (two threads per
@@ -367,7 +368,9 @@ zinv_panel_kernel(double2* S, int64_t sS, int n, int k, int nbe, char* aux, int6
 // through the wave's own LDS area into the row layout and back, without a barrier.
 //  * pivot key: high word of |re| + |im| with the row in its low bits (10 of its 20
 //    mantissa bits decide, the first row on ties), so that a wave's maximum is four
-//    32-bit DPP steps and one word says key, row and wave;
+//    32-bit DPP steps and one word says key, row and wave.  A pivot up to 0.1% below the
+//    largest entry costs no accuracy (rms error of the selected solve against 64 bits, whole keys / these: 48 rows
+//    1.77e-14 / 1.67e-14, 77 1.68e-14 / 1.72e-14, 128 2.06e-14 / 2.06e-14, 512 1.18e-14 / 1.17e-14);
 //  * two barriers per step: the waves' keys before the first, and only the winning row
 //    is written, before the second (one lane's 8 writes: 264 cycles, by four waves at
 //    once 468);
